@@ -144,6 +144,16 @@ int tml_hip_sgemm_q8(int64_t M, int64_t N, int64_t K, const float *A, const int8
  * taken from x clamped to the largest finite bf16, so a finite x near
  * FLT_MAX keeps a finite product where q is 0 or +-1. */
 
+/* Arithmetic of the f32, F16 and Q8_K products past the decoder rows (every
+ * entry point): fp32 multiply-adds on the fp32 matrix cores, or -- where that is
+ * faster, the larger products -- the bf16 matrix cores with every operand split
+ * exactly into bf16 terms and the products of the terms summed in fp32, dropped
+ * terms below 2^-25 of a product; both are fp32 results (2-norm error against 64
+ * bits 1e-7 to 1e-6).  Infinities, NaNs, values past the largest bf16 and sums
+ * below 2^-70 are recomputed as ascending fp32 sums.  Limit: where one operand
+ * is past 2^22 in magnitude, the other's elements below 2^-109 are taken to an
+ * absolute 2^-134. */
+
 /* C = A . dequant(Q8_K B).  Replaces zblas.sgemmQ8K(m, n, k, a, b.data,
  * b.scales, b.block_size, c) at src/core/quantization.zig:555
  * (matmulF32Q8KSimd, :528-617).  scales holds ceil(K*N/block) values;

@@ -231,6 +231,7 @@ tml_emu_launcher<P...> tml_emu_launch(void (*k)(P...), dim3 g, dim3 b, size_t sh
 
 // ------------------------------------------------------------- device side
 inline void __syncthreads() {}
+inline int __syncthreads_or(int v) { return v; }
 template <typename A, typename B>
 inline std::common_type_t<A, B> min(A a, B b) {
     return a < b ? a : b;
@@ -274,6 +275,7 @@ typedef uint32_t tml_emu_u32x2 __attribute__((ext_vector_type(2)));
 inline void __builtin_amdgcn_s_waitcnt(int) {}
 inline void __builtin_amdgcn_s_barrier() {}
 inline void __builtin_amdgcn_sched_barrier(int) {}
+inline void __builtin_amdgcn_sched_group_barrier(int, int, int) {}
 inline void __builtin_amdgcn_wave_barrier() {}
 inline void __builtin_amdgcn_fence(int, const char *) {}
 template <typename T>

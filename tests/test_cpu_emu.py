@@ -325,3 +325,24 @@ def test_noalloc_entry_point(emu):
     assert len(_ok_lines(outs)) == len(ok_cases), _err_lines(outs)
     outs, fails = run_cases(emu, ["noalloc 0 512 1024 4096 - TML_GEMM_SPLIT=8"], workers=1)
     assert not fails and len(_err_lines(outs)) == 1 and "static scratch" in _err_lines(outs)[0]
+
+
+def test_sbf_cases(emu):
+    # the split-bf16 GEMM (TML_GEMM_SBF_TILE 1-5): every tile and format on shapes
+    # ragged in M, N and K, odd N, the smallest K, every epilogue; the planner's
+    # own choice at encoder sizes; and a short operand, which must be reported
+    cases = []
+    for tile in range(1, 6):
+        env = f"TML_GEMM_SBF_TILE={tile}"
+        for fmt, shapes in [(F32, [(200, 324, 516), (33, 131, 40), (9, 77, 4), (257, 129, 36)]),
+                            (F16, [(200, 328, 520), (33, 131, 40), (300, 70, 1288)]),
+                            (Q8_K, [(200, 352, 516), (33, 128, 40), (300, 64, 1288)])]:
+            for (M, N, K) in shapes:
+                cases += [f"gemm {fmt} {M} {N} {K} br {env}", f"gemm {fmt} {M} {N} {K} teB {env}"]
+    cases += ["gemm 0 1500 3840 64 b", "gemm 4 1500 3840 64 e", "gemm 3 1500 3840 64 br", "gemm 0 100 1001 388 bt"]
+    outs, fails = run_cases(emu, cases)
+    assert not fails and not _err_lines(outs), (fails, _err_lines(outs)[:3])
+    assert len(_ok_lines(outs)) == len(cases)
+    for fmt in (F32, F16, Q8_K):
+        _, fails = run_cases(emu, [f"gemm {fmt} 200 352 512 S TML_GEMM_SBF_TILE=2"], workers=1)
+        assert fails, f"the CPU build did not report a short operand of format {fmt}"

@@ -1,0 +1,133 @@
+"""The split-bf16 GEMM (gemm_sbf.hip: f32 / F16 / Q8_K weights, M > 8) against 64-bit products.
+
+Every operand is split exactly into bf16 terms and the products of the terms
+that matter are summed in fp32, so an output differs from the 64-bit product
+of the same operands by at most one fp32 rounding of each 32-deep slice's sum,
+the six dropped or merged small terms (below 2^-24 of a product together) and
+the epilogue's own roundings:
+    |C - ref| <= (ceil(K / 32) + 8) * 2^-24 * sum_k |a b| + 2^-23 |ref|.
+Operands the split does not carry (infinities, NaNs, values past the largest
+bf16, sums of products below 2^-70) are recomputed in fp32 in ascending k, as
+the reference does (src/core/ops.zig:277-414), so their inf / NaN pattern is the
+oracle's.  TML_GEMM_SBF_TILE picks a tile, TML_GEMM_SBF=0 turns the kernel off.
+"""
+import os
+
+import numpy as np
+import pytest
+
+from tomoul_amd import _abi, synth
+
+pytestmark = pytest.mark.gpu
+TILES = (1, 2, 3, 4, 5)
+
+
+@pytest.fixture
+def env():
+    keys = ("TML_GEMM_SBF_TILE", "TML_GEMM_SBF")
+    saved = {key: os.environ.get(key) for key in keys}
+    yield os.environ
+    for key, v in saved.items():
+        if v is None:
+            os.environ.pop(key, None)
+        else:
+            os.environ[key] = v
+
+
+def weight(orc, fmt, w):
+    """(bytes, scales, the fp32 values [K,N]) of w in format fmt."""
+    if fmt == _abi.FMT_F32:
+        return w, None, w
+    if fmt == _abi.FMT_F16:
+        h = orc.to_f16(w)
+        return h, None, h.view(np.float16).astype(np.float32).reshape(w.shape)
+    q, s = orc.quantize_q8k(w)
+    flat = np.repeat(s, 32)[: w.size] * q.reshape(-1).astype(np.float32)
+    return q, s, flat.astype(np.float32).reshape(w.shape)
+
+
+def run(fmt, m, n, k, a, q, scales, **kw):
+    c = np.zeros((m, n), np.float32)
+    _abi.gemm(fmt, m, n, k, a, np.ascontiguousarray(q), c, scales=scales, **kw)
+    return c
+
+
+def check(c, a, w, bias=None, res=None):
+    ref = a.astype(np.float64) @ w.astype(np.float64)
+    mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64)
+    bound = (-(-a.shape[1] // 32) + 8) * 2.0**-24 * mag
+    for x in (bias, res):
+        if x is not None:
+            ref = ref + x
+            bound = bound + 2.0**-24 * (np.abs(ref) + np.abs(x))
+    worst = float(np.max(np.abs(c - ref) / (bound + 2.0**-23 * np.abs(ref) + 1e-300)))
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("fmt", [_abi.FMT_F32, _abi.FMT_F16, _abi.FMT_Q8_K])
+@pytest.mark.parametrize("tile", TILES)
+def test_sbf_tiles(orc, env, tile, fmt):
+    # partial tiles in M and N, one slice to many, K not a whole slice
+    env["TML_GEMM_SBF_TILE"] = str(tile)
+    for (m, n, k) in [(9, 32, 4), (33, 160, 36), (257, 288, 520), (130, 96, 1032)]:
+        if fmt != _abi.FMT_Q8_K:
+            n += 1  # odd rows: the scalar stores, unaligned B rows
+        a, bias = synth.normal_matrix(11 + m, m, k), synth.normal(12, n, 0.0, 0.02)
+        q, scales, w = weight(orc, fmt, synth.normal_matrix(13, k, n, 0.02))
+        check(run(fmt, m, n, k, a, q, scales, bias=bias), a, w, bias.astype(np.float64))
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [(_abi.FMT_F32, 300, 5120, 1280), (_abi.FMT_F16, 700, 2048, 640),
+                                       (_abi.FMT_Q8_K, 900, 3072, 768), (_abi.FMT_F32, 77, 1001, 388)])
+def test_sbf_default_plan_epilogue(orc, fmt, m, n, k):
+    # the planner's own choice, with the residual and both activations
+    a, bias, res = synth.normal_matrix(21, m, k), synth.normal(22, n, 0.0, 0.02), synth.normal_matrix(23, m, n)
+    q, scales, w = weight(orc, fmt, synth.normal_matrix(24, k, n, 0.02))
+    c = np.zeros((m, n), np.float32)
+    _abi.gemm_residual(fmt, m, n, k, a, q, res, c, scales=scales, bias=bias)
+    check(c, a, w, bias.astype(np.float64), res.astype(np.float64))
+    plain = run(fmt, m, n, k, a, q, scales, bias=bias)
+    for act, gelu in ((_abi.ACT_GELU_ERF, orc.gelu_exact), (_abi.ACT_GELU_TANH, orc.gelu_tanh)):
+        _abi.gemm_act(fmt, m, n, k, a, q, c, act=act, scales=scales, bias=bias)
+        ref = gelu(plain)
+        assert np.max(np.abs(c - ref)) <= 1e-6 * max(1.0, np.max(np.abs(ref))), act
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_sbf_inf_nan(orc, env, tile):
+    env["TML_GEMM_SBF_TILE"] = str(tile)
+    m, n, k = 140, 100, 100  # K is no whole slice: row r's tail reads row r + 1's head
+    a, w = synth.normal_matrix(31, m, k), synth.normal_matrix(32, k, n, 0.02)
+    a[3, 5], a[4, 0], a[64, 99], a[139, 7] = np.inf, -np.inf, np.nan, np.float32(3.4028235e38)
+    w[5, 9], w[7, 10], w[11, 20], w[12, 21] = 0.0, 0.0, np.inf, np.nan
+    a[70, 11] = 0.0
+    c, ref = run(_abi.FMT_F32, m, n, k, a, w, None), orc.matmul(a, w)
+    assert np.array_equal(np.isnan(c), np.isnan(ref)) and np.array_equal(np.isposinf(c), np.isposinf(ref))
+    assert np.array_equal(np.isneginf(c), np.isneginf(ref))
+    fin = np.isfinite(ref)
+    # the recomputed sums and the others alike, 100 terms
+    mag = np.where(np.isfinite(a), np.abs(a), 0).astype(np.float64) @ np.where(np.isfinite(w), np.abs(w), 0)
+    assert np.all(np.abs(c[fin].astype(np.float64) - ref[fin]) <= 2.0**-23 * 100 * mag[fin])
+
+
+@pytest.mark.parametrize("scale", [2.0**-100, 2.0**-60, 2.0**60, 2.0**110])
+def test_sbf_range(env, scale):
+    # the whole exponent range of A: a power of two times the operand is the same
+    # power times the result, also where the third term falls under bf16's
+    # denormals (there the sum is recomputed in fp32: K roundings)
+    env["TML_GEMM_SBF_TILE"] = "5"
+    m, n, k = 70, 65, 96
+    a, w = synth.normal_matrix(41, m, k), synth.normal_matrix(42, k, n, 0.02)
+    c = run(_abi.FMT_F32, m, n, k, a * np.float32(scale), w, None).astype(np.float64) / scale
+    ref = a.astype(np.float64) @ w.astype(np.float64)
+    mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64)
+    assert np.max(np.abs(c - ref) / mag) <= k * 2.0**-24
+
+
+def test_sbf_exact_integers(env):
+    # products and sums of small integers are exact
+    rng = np.random.default_rng(5)
+    a, w = rng.integers(-999, 1000, (200, 320)).astype(np.float32), rng.integers(-9, 10, (320, 129)).astype(np.float32)
+    for tile in TILES:
+        env["TML_GEMM_SBF_TILE"] = str(tile)
+        assert np.array_equal(run(_abi.FMT_F32, 200, 129, 320, a, w, None), a @ w)

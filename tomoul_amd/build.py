@@ -17,7 +17,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libtomoul_hip.so")
-SOURCES = ["runtime.hip", "gemm_mfma.hip", "gemm_dma.hip", "gemm_qbf.hip", "gemv.hip", "gemv_t.hip", "gemv_tm.hip", "quantize.hip", "tl.hip",
+SOURCES = ["runtime.hip", "gemm_mfma.hip", "gemm_dma.hip", "gemm_qbf.hip", "gemm_sbf.hip", "gemv.hip", "gemv_t.hip", "gemv_tm.hip", "quantize.hip", "tl.hip",
            "stream_read.hip", "gemv_x.hip"]
 ARCH = os.environ.get("TML_OFFLOAD_ARCH", "gfx950")
 
@@ -40,10 +40,10 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found: the HIP backend cannot be built")
 
 
-# Per-source flags.  gemm_qbf.hip: keep MFMA accumulators in ordinary VGPRs
+# Per-source flags.  gemm_qbf.hip, gemm_sbf.hip: keep MFMA accumulators in ordinary VGPRs
 # (the compiler otherwise splits them over the accumulation registers and
 # copies them back and forth inside the K loop: 72 extra moves a loop trip).
-SOURCE_FLAGS = {"gemm_qbf.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+SOURCE_FLAGS = {src: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for src in ("gemm_qbf.hip", "gemm_sbf.hip")}
 
 
 def _compile(src: str, obj_dir: str) -> str:

@@ -512,7 +512,8 @@ int device_cus() {
 // 512x4096x768 34.39 / 40.17 -> 32.82 / 37.56, 384x4096x1024 34.93 / 41.19
 // -> 33.23 / 37.17, 512x3072x768 Q8_K 32.54 -> 30.85, 1500x3840x1280
 // 134.1 / 150.2 -> 130.7 / 142.6.  Q4_0 and Q8_0 keep the f32 table.
-void pick_dma(int64_t M, int64_t N, int64_t K, int fmt, GemmPlan *p) {
+// Returns the plan's modelled time (infinite for a forced split too deep for K).
+double pick_dma(int64_t M, int64_t N, int64_t K, int fmt, GemmPlan *p) {
     static const double f32_one[] = {1.975, 0.974, 0.528, 4.05, 1.06, 0.54, 0.308, 0.308, 0.354, 0.226, 0.165};
     static const double f32_many[] = {1.998, 0.854, 0.504, 4.05, 1.147, 0.672, 0.24, 0.293, 0.383, 0.282, 0.155};
     static const double f16_one[] = {2.40, 1.276, 0.680, 4.66, 1.162, 0.690, 0.418, 0.396, 0.556, 0.359, 0.21};
@@ -602,6 +603,7 @@ void pick_dma(int64_t M, int64_t N, int64_t K, int fmt, GemmPlan *p) {
     // headline step than the extra launch (the agent-scope round trip of the
     // last split costs more than a reduce kernel in a graph), so it is off.
     p->fused = p->nsplit > 1 && env_int("TML_GEMM_FUSED", 0) != 0 && gemm_dma_cfg_fusable(p->cfg);
+    return best_t;
 }
 
 bool aligned(const void *p, size_t n) { return ((uintptr_t)p % n) == 0; }
@@ -692,12 +694,28 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
         const int64_t tiles = ((m.M + kCfgs[c].bm - 1) / kCfgs[c].bm) * ((m.N + kCfgs[c].bn - 1) / kCfgs[c].bn);
         few_tiles = tiles < cus / 2 || (tiles < cus && m.K >= 2048);
     }
+    double other_us = 1e300;  // modelled time of the fp32-MFMA plan
     const bool by_m = m.fmt == TML_FMT_F16 || (m.fmt == TML_FMT_Q8_K && !(m.M >= 512 && m.N >= 4096)) ||
                       (m.fmt == TML_FMT_Q4_0 && (m.M >= 1024 || m.M <= 128));
     const bool narrow_ok = m.fmt == TML_FMT_F32 || dma_q == 1 || (dma_q < 0 && (by_m || few_tiles));
     if (narrow_ok && env_int("TML_GEMM_DMA", 1) != 0 && gemm_dma_supported(m) && m.K > 0) {
         p.dma = true;
-        pick_dma(m.M, m.N, m.K, m.fmt, &p);
+        other_us = pick_dma(m.M, m.N, m.K, m.fmt, &p);
+    } else if (gemm_dma_supported(m) && m.K > 0) {
+        // the register-staged kernel, within a few per cent of the direct-copy
+        // one where it is preferred
+        GemmPlan unused;
+        other_us = pick_dma(m.M, m.N, m.K, m.fmt, &unused);
+    }
+    // f32, F16 and Q8_K where the split-bf16 kernel is modelled faster (or
+    // neither of the two above has a fast path, e.g. odd N), unless an override
+    // asks for one of the fp32-MFMA kernels.
+    const bool other_forced = fp32_forced || set("TML_GEMM_DMA") || set("TML_GEMM_FUSED") || set("TML_GEMM_XCDPART") ||
+                              set("TML_GEMM_XCD") || set("TML_GEMM_GROUPM");
+    GemmPlan q;
+    if (!other_forced && gemm_sbf_supported(m) && pick_sbf(m, other_us, &q)) {
+        q.sbf = true;
+        return q;
     }
     return p;
 }
@@ -751,6 +769,7 @@ Status launch_gemm_mfma(const MatmulArgs &m, const Workspace &ws, hipStream_t s)
     // TML_REQUIRE_SPLIT=1 (tests): refuse a plan that does not split K
     if (!((p.qbf || p.dma) && p.nsplit > 1) && env_int("TML_REQUIRE_SPLIT", 0) == 1)
         return Status::Err(TML_ERR_INVALID_ARG, "TML_REQUIRE_SPLIT=1: this call's plan does not split K");
+    if (p.sbf) return launch_gemm_sbf(m, p, s);
     if (p.qbf) return launch_gemm_qbf(m, p, ws, s);
     if (p.dma) return launch_gemm_f32_dma(m, p, ws, s);
     const int cus = device_cus();

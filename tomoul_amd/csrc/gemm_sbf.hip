@@ -1,0 +1,659 @@
+// gemm_sbf.hip -- f32 / F16 / Q8_K GEMM on the bf16 matrix cores, every
+// operand split exactly into bf16 terms.
+//
+//   C[M,N] = act(alpha * A[M,K] . B[K,N] + beta * C + bias[N] + R)
+//
+// The reference's products are fp32 (src/core/ops.zig:277-414; f16 and Q8_K
+// weights widened to f32, src/core/quantization.zig:559-614, :1921-1962).  An
+// fp32 value's 24 bits are three bf16 terms, x = h + m + l, each the nearest
+// bf16 of what the ones before leave (|m| <= 2^-9 |x|, |l| <= 2^-18 |x|, the
+// sum exact), so
+//   a . b = hh + hm + mh + mm + hl + lh  (+ ml + lm + ll, at most 2^-25 |a b|)
+// with every kept product exact.  Six v_mfma_f32_16x16x32_bf16 (five for f16
+// weights, whose 11 bits are two bf16 terms, h + m, exactly) do the work of eight
+// v_mfma_f32_16x16x4_f32 at 16 times their rate: 2.5 PFLOP/s / 6 = 417 against 157
+// TFLOP/s.  The dropped terms are below half an fp32 rounding of the product, and
+// the hh products have an accumulator of their own, which a 32-deep slice rounds
+// once where the fp32 matrix cores round theirs eight times: the 2-norm error
+// against 64 bits is 0.9e-7 - 4.5e-7 over the shapes at pick_sbf, theirs 3.7e-7 -
+// 9.9e-7.
+//
+// Bound: the matrix cores, at the clock the power limit leaves them.  At
+// 1500x5120x1280 (240 tiles of 256x128) the main loop keeps them 82 % busy, at
+// 1.85 GHz (2.3 GHz with 48 CUs busy): 95 us, 207 TFLOP/s, 165 us before on the
+// fp32 matrix cores.
+//
+// Values the split does not carry -- infinities and NaNs (their residual is
+// NaN), |x| above the largest bf16, and magnitudes so small that l falls under
+// bf16's denormals (|x| < 2^-109) -- show in the sum: it is not finite, or not
+// zero and below 2^-70.  The epilogue recomputes such an output from the
+// operands as an ascending fp32 sum, the reference's own.
+#include "tml_internal.hpp"
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+namespace tml {
+namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+constexpr int kSbfXcd = 8;  // XCDs of an MI355X: workgroups are dealt to them round robin
+
+struct SbfArgs {
+    int M, N, K;
+    const float *A;         // [M,K], K % 4 == 0, 16-byte aligned
+    const uint8_t *B;       // [K,N]: f32, binary16 or int8
+    const float *scales;    // Q8_K block scales (32 elements each, N % 32 == 0)
+    int ldb;                // bytes per B row
+    const float *bias;      // [N] or nullptr
+    const float *res;       // [M,N] residual after the bias, or nullptr (may equal C)
+    float *C;
+    float alpha, beta;
+    int act;
+    long long tail0;
+    unsigned a_bytes, b_bytes, s_bytes;  // M * K * 4, K * ldb, scale bytes
+    int tiles_m, tiles_n;
+    int vec_epi;            // N % 4 == 0 and C, bias, residual 16-byte aligned
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sbf_rsrc(const void *base, unsigned nbytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)nbytes, 0x00020000);
+}
+
+// Two floats to two bf16 (round to nearest even), a in the low half.
+__device__ __forceinline__ uint32_t sbf_pk(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){a, b}, bf16x2));
+}
+// NP bf16 terms of a pair of values.
+template <int NP>
+__device__ __forceinline__ void sbf_split(float a, float b, uint32_t (&t)[NP]) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        t[p] = sbf_pk(a, b);
+        if (p + 1 < NP) {
+            a -= __uint_as_float(t[p] << 16);
+            b -= __uint_as_float(t[p] & 0xFFFF0000u);
+        }
+    }
+}
+
+// Physical slot of logical slot s (8 k) in LDS row r of SL slots: four
+// slots (64-byte rows) swap by (r / 2) mod 4, eight (128-byte rows) by r mod 8,
+// so that the operand reads (16 rows, one slot each four lanes apart) and the
+// staging writes (64 rows, one slot) run at the LDS's full rate: measured 8.3 and
+// 13.9 cycles a 16-byte wave access, (r / 4) mod 4 9.3 and 16.3.
+template <int SL>
+__device__ __forceinline__ int sbf_slot(int r, int s) {
+    if constexpr (SL == 4) return r * 4 + (s ^ ((r >> 1) & 3));
+    else return r * 8 + (s ^ (r & 7));
+}
+
+// bf16 terms of B: a binary16 weight is two exactly.
+template <int FMT>
+constexpr int kSbfPlanesB = FMT == TML_FMT_F16 ? 2 : 3;
+
+// One element of B as the f32 the reference multiplies by.
+template <int FMT>
+__device__ __forceinline__ float sbf_b(const SbfArgs &a, int k, int n) {
+    if constexpr (FMT == TML_FMT_F32) return ((const float *)a.B)[(size_t)k * a.N + n];
+    else if constexpr (FMT == TML_FMT_F16) return tml_half_bits(((const uint16_t *)a.B)[(size_t)k * a.N + n]);
+    else return (float)((const int8_t *)a.B)[(size_t)k * a.N + n] * a.scales[((size_t)k * a.N + n) >> 5];
+}
+
+// A sum that shows operands the split does not carry (top of the file).
+__device__ __forceinline__ bool sbf_suspect(float v) {
+    const uint32_t u = __float_as_uint(v) & 0x7FFFFFFFu;
+    return u - 1u >= 0x7F7FFFFFu || u - 1u < 0x1C7FFFFFu ? u != 0u : false;  // not finite, or 0 < |v| < 2^-70
+}
+// The ascending fp32 sum of output (row, col)'s products.
+template <int FMT>
+__device__ __forceinline__ float sbf_fp32_sum(const SbfArgs &a, int row, int col) {
+    float s = 0.0f;
+    for (int k = 0; k < a.K; ++k) s = fmaf(a.A[(size_t)row * a.K + k], sbf_b<FMT>(a, k, col), s);
+    return s;
+}
+
+// A workgroup of NW = 4 or 8 waves owns a BM x BN tile of C, each wave a WM x
+// WN sub-tile (or, with KW = 2 wave groups, half the k of one), and walks K in
+// BK-deep slices.  A wave loads the A it multiplies straight into registers, in
+// the MFMA's own layout, and splits it there; B is loaded once per workgroup,
+// split, and passed through three LDS stages as rows of 16-byte slots (8 k), one
+// barrier a slice: a slice is written two steps before it is multiplied, so its
+// first operands are read before the barrier that starts its step.  (With A in LDS too, its writes -- 64 bytes a clock -- and
+// reads took the LDS as long as the products take the matrix cores.)  Slices are
+// loaded D ahead, and the splitting of the next slice is dealt out between the
+// groups of matrix instructions of this one: VALU work in the wave that waits on
+// the matrix core is nearly free, the same work in another wave is not (measured:
+// 16 MFMAs and 32 subtractions a wave, two waves a SIMD, 690 cycles interleaved,
+// 615 without the subtractions; half the waves on each, the sum of the two).
+//
+// k order: slot g of a 32-k half holds k = 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4
+// g + 3, so that each of a lane's two 16-byte A loads covers 64 contiguous bytes
+// of a row over its four lanes.
+template <int FMT, int BM, int BN, int WM, int WN, int BK, int KW, int NW, int D>
+__global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
+    static_assert(KW == 1 ? BK == 32 : KW == 2 && BK == 64, "each wave group multiplies one 32-k half of a slice");
+    static_assert(NW == 4 || NW == 8, "one or two waves a SIMD");
+    constexpr int NA = 3, NB = kSbfPlanesB<FMT>;
+    constexpr int SL = BK / 8;    // 16-byte slots (8 k) of an LDS row
+    constexpr int NT = 64 * NW;
+    constexpr int NWS = NW / KW;  // waves per group, one per sub-tile
+    constexpr int TM = WM / 16, TN = WN / 16, WAVES_N = BN / WN;
+    static_assert((BM / WM) * (BN / WN) == NWS, "one wave of a group per WM x WN sub-tile");
+    // B's staging tasks: one (column, 8-k slot) each, PB a thread.
+    constexpr int TB = BN * SL, PB = (TB + NT - 1) / NT;
+    constexpr int RW = FMT == TML_FMT_Q8_K ? 16 : 8;  // registers of a task (Q8_K: 8 values, 8 scales)
+
+    constexpr int kStage = BN * SL * NB;  // 16-byte slots of a stage
+    constexpr int CS = BN + 4;            // floats of a staged C row (rows 4 apart: 16 banks on)
+    constexpr int kLds = 3 * kStage > BM * CS / 4 ? 3 * kStage : BM * CS / 4;
+    __shared__ uintx4 lds[kLds];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = KW == 2 ? wave / NWS : 0;
+    const int sw = wave % NWS;
+    const int wm0 = (sw / WAVES_N) * WM, wn0 = (sw % WAVES_N) * WN;
+    const int c = lane & 15, g = lane >> 4;
+
+    // Workgroup -> tile: consecutive ids within each XCD (own L2), in groups
+    // of eight tile rows so that neighbours share A rows and B columns.
+    int tile_m, tile_n;
+    {
+        const int nblk = gridDim.x, b = blockIdx.x;
+        const int per = nblk / kSbfXcd, rem = nblk % kSbfXcd;
+        const int xcd = b % kSbfXcd, idx = b / kSbfXcd;
+        const int lin = (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+        constexpr int GM = 8;
+        const int group = GM * a.tiles_n;
+        const int first_m = (lin / group) * GM;
+        const int gsize = min(a.tiles_m - first_m, GM);
+        tile_m = first_m + (lin % group) % gsize;
+        tile_n = (lin % group) / gsize;
+    }
+    const int m0 = tile_m * BM, n0 = tile_n * BN;
+
+    // ---- loads.  A lane's offsets are fixed; the slice moves the buffer's base
+    // and byte count (scalar work only).  Rows of A past M and k-rows of B past K
+    // lie past the byte count and read zeros.  A's k past K reads the next row,
+    // against B's zero rows; B columns past N read the next k-row and feed dropped
+    // outputs.  (A value there that is not finite makes its sum a NaN, which the
+    // epilogue recomputes.)
+    constexpr unsigned ESZ = FMT == TML_FMT_F32 ? 4u : FMT == TML_FMT_F16 ? 2u : 1u;
+    const unsigned a_off = ((unsigned)c * (unsigned)a.K + 4u * (unsigned)g) * 4u;
+    unsigned b_off[PB], s_off[PB];
+    int slot_b[PB];
+#pragma unroll
+    for (int t = 0; t < PB; ++t) {
+        const int j = tid + t * NT, n = j % BN, sl = j / BN;
+        const unsigned k = (unsigned)(32 * (sl / 4) + 4 * (sl % 4));
+        b_off[t] = k * (unsigned)a.ldb + (unsigned)n * ESZ;
+        s_off[t] = k * ((unsigned)a.N / 8u) + (unsigned)n / 32u * 4u;
+        slot_b[t] = sbf_slot<SL>(n, sl % SL);
+    }
+    auto moved = [](const void *base, unsigned nbytes, unsigned adv) __attribute__((always_inline)) {
+        adv = min(adv, nbytes);
+        return sbf_rsrc((const char *)base + adv, nbytes - adv);
+    };
+    // the buffers at a slice's first k
+    auto at_a = [&](int k0) __attribute__((always_inline)) {
+        return moved(a.A, a.a_bytes, ((unsigned)(m0 + wm0) * (unsigned)a.K + (unsigned)(k0 + 32 * kg)) * 4u);
+    };
+    auto at_b = [&](int k0) __attribute__((always_inline)) {
+        return moved(a.B, a.b_bytes, (unsigned)k0 * (unsigned)a.ldb + (unsigned)n0 * ESZ);
+    };
+    auto at_s = [&](int k0) __attribute__((always_inline)) {  // scale of (k, n): scales[k * N / 32 + n / 32]
+        return FMT == TML_FMT_Q8_K ? moved(a.scales, a.s_bytes, (unsigned)k0 * ((unsigned)a.N / 8u) + (unsigned)n0 / 8u)
+                                   : sbf_rsrc(a.B, 0u);
+    };
+    uint32_t ra[D][TM][8], rb[D][PB][RW];
+    // half h of A tile i's eight k, and k-row kk of B task t
+    // (off: the lane's offset, from fresh() -- a sum the compiler cannot keep in a
+    // register per row over the whole loop, where there is none to spare)
+    auto fresh = [](unsigned off) __attribute__((always_inline)) {
+        __asm__ volatile("" : "+v"(off));
+        return off;
+    };
+    auto load_a = [&](__amdgpu_buffer_rsrc_t rs, unsigned off, int i, int h, int d) __attribute__((always_inline)) {
+        const uintx4 v =
+            __builtin_amdgcn_raw_buffer_load_b128(rs, off + (unsigned)(16 * i) * (unsigned)a.K * 4u + 64u * h, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ra[d][i][4 * h + e] = v[e];
+    };
+    auto load_b = [&](__amdgpu_buffer_rsrc_t rs, __amdgpu_buffer_rsrc_t rsc, unsigned off0, int t, int kk, int d)
+                      __attribute__((always_inline)) {
+        const unsigned row = (unsigned)((kk < 4 ? 0 : 12) + kk);
+        const unsigned off = off0 + row * (unsigned)a.ldb;
+        if constexpr (FMT == TML_FMT_F32) rb[d][t][kk] = __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
+        else if constexpr (FMT == TML_FMT_F16) rb[d][t][kk] = __builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0);
+        else {
+            rb[d][t][kk] = __builtin_amdgcn_raw_buffer_load_b8(rs, off, 0, 0);
+            rb[d][t][8 + kk] = __builtin_amdgcn_raw_buffer_load_b32(rsc, s_off[t] + row * ((unsigned)a.N / 8u), 0, 0);
+        }
+    };
+
+    // ---- splitting, a pair of k at a time: A's pair e to word e of the next
+    // slice's operands, B's to word e of the slots write_b stores.
+    uintx4 av[2][NA][TM], bp[PB][NB];
+    auto split_a = [&](int i, int e, int d, int nxt) __attribute__((always_inline)) {
+        uint32_t t[NA];
+        sbf_split<NA>(__uint_as_float(ra[d][i][2 * e]), __uint_as_float(ra[d][i][2 * e + 1]), t);
+#pragma unroll
+        for (int p = 0; p < NA; ++p) av[nxt][p][i][e] = t[p];
+    };
+    auto split_b = [&](int t, int e, int d) __attribute__((always_inline)) {
+#pragma clang fp contract(off)  // (the dequantized value is the rounded product, in every tile)
+        float x[2];
+#pragma unroll
+        for (int z = 0; z < 2; ++z) {
+            const uint32_t w = rb[d][t][2 * e + z];
+            if constexpr (FMT == TML_FMT_F32) x[z] = __uint_as_float(w);
+            else if constexpr (FMT == TML_FMT_F16) x[z] = tml_half_bits(w);
+            else x[z] = (float)(int8_t)w * __uint_as_float(rb[d][t][8 + 2 * e + z]);
+        }
+        uint32_t v[NB];
+        sbf_split<NB>(x[0], x[1], v);
+#pragma unroll
+        for (int p = 0; p < NB; ++p) bp[t][p][e] = v[p];
+    };
+    auto write_b = [&](int t, int p, int stage) __attribute__((always_inline)) {
+        if (TB % NT == 0 || tid + t * NT < TB) lds[stage + slot_b[t] + p * BN * SL] = bp[t][p];
+    };
+
+    // acc holds the hh products, cor the five (four) smaller ones: a slice
+    // rounds the large sum once, and the small terms keep their own.
+    floatx4 acc[TM][TN], cor[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = cor[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+
+    // One slice: A's operands av[cur] and the LDS stage at sr are multiplied,
+    // while B's register set db becomes the stage at sw (two slices on) and A's
+    // set da becomes av[nxt] (the next slice).  Lane (c, g) reads slot g (of its
+    // group's half) of B columns wn0 + 16 j + c.  JB columns at a time, plane pair
+    // by plane pair: a group of TM * JB MFMAs is independent, and a share of the
+    // staging follows each group.  A B plane's registers take the next columns --
+    // after the last, the first of the next slice at sn -- as soon as the last
+    // product that needs it has run.
+    constexpr int NP = NB == 3 ? 6 : 5, JB = TM >= 4 ? 1 : TM >= 2 || TN < 4 ? 2 : 4, kGroups = TN / JB * NP;
+    static_assert(TN % JB == 0, "whole groups of columns");
+    uintx4 bv[NB][JB];
+    const int slot_r = sbf_slot<SL>(wn0 + c, 4 * kg + g);
+    auto read_b = [&](int p, int j0, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < JB; ++j) bv[p][j] = lds[stage + slot_r + p * BN * SL + 16 * SL * (j0 + j)];
+    };
+    // When the staging runs: splitting step v (B's tasks, then A's tiles, four
+    // pairs each) after group v kGroups / kSplits; a task's or tile's reloads from
+    // the group after its last pair on, two k-rows or one half a group, and B's
+    // plane writes every few groups: bunched, the writes hold up the operand reads
+    // behind them and the loads' issue holds up the wave.
+    constexpr int kSplits = 4 * (PB + TM);
+    auto split_at = [](int v) constexpr { return v * kGroups / kSplits; };
+    auto load_at = [](int task, int i) constexpr {
+        const int g0 = (4 * task + 3) * kGroups / kSplits + i;
+        return g0 < kGroups ? g0 : kGroups - 1;
+    };
+    auto write_at = [](int t, int p) constexpr {
+        const int g0 = (4 * t + 3) * kGroups / kSplits;
+        return g0 + (kGroups - 1 - g0) * p / NB;
+    };
+    auto slice = [&](int cur, int nxt, int sr, int sn, int sw_, int db, int kb, int da,
+                     int ka) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rsa = at_a(ka), rsb = at_b(kb), rss = at_s(kb);
+        const unsigned a_fresh = fresh(a_off);
+        unsigned b_fresh[PB];
+#pragma unroll
+        for (int w = 0; w < PB; ++w) b_fresh[w] = fresh(b_off[w]);
+#pragma unroll
+        for (int j0 = 0; j0 < TN; j0 += JB) {
+            constexpr int QA[6] = {0, 1, 2, 0, 1, 0}, QB[6] = {0, 0, 0, 1, 1, 2};
+#pragma unroll
+            for (int t = 0; t < NP; ++t) {
+#pragma unroll
+                for (int j = 0; j < JB; ++j)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        floatx4 &to = t == 0 ? acc[i][j0 + j] : cor[i][j0 + j];
+                        to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[cur][QA[t]][i]),
+                                                                     __builtin_bit_cast(bf16x8, bv[QB[t]][j]), to, 0,
+                                                                     0, 0);
+                    }
+                if (t + 1 == NP || QB[t + 1] != QB[t]) {
+                    if (j0 + JB < TN) read_b(QB[t], j0 + JB, sr);
+                    else read_b(QB[t], 0, sn);
+                }
+                const int gi = j0 / JB * NP + t;
+#pragma unroll
+                for (int v = 0; v < kSplits; ++v)
+                    if (split_at(v) == gi) {
+                        if (v < 4 * PB) split_b(v / 4, v % 4, db);
+                        else split_a(v / 4 - PB, v % 4, da, nxt);
+                    }
+#pragma unroll
+                for (int w = 0; w < PB; ++w) {
+#pragma unroll
+                    for (int kk = 0; kk < 8; ++kk)
+                        if (load_at(w, kk / 2) == gi) load_b(rsb, rss, b_fresh[w], w, kk, db);
+#pragma unroll
+                    for (int p = 0; p < NB; ++p)
+                        if (write_at(w, p) == gi) write_b(w, p, sw_);
+                }
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        if (load_at(PB + i, h) == gi) load_a(rsa, a_fresh, i, h, da);
+#pragma unroll
+                for (int i = 0; i < TM * JB; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+
+    // Register sets d hold the slices kt with kt % D == d.  In step kt, A's set
+    // (kt + 1) % D becomes av and takes slice kt + 1 + D, B's set (kt + 2) % D
+    // becomes the stage (kt + 2) % 3 and takes slice kt + 2 + D.  The step count
+    // is rounded up to whole rounds of U = lcm(2, D) steps (steps past K multiply
+    // zeros), so a step's register sets are fixed in the code.
+    constexpr int U = D % 2 == 0 ? D : 2 * D;
+    const int nk = ((a.K + BK - 1) / BK + U - 1) / U * U;
+    auto barrier = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    auto load_set = [&](bool is_a, int d, int k0) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t rsa = at_a(k0), rsb = at_b(k0), rss = at_s(k0);
+#pragma unroll
+        for (int t = 0; t < PB && !is_a; ++t)
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) load_b(rsb, rss, b_off[t], t, kk, d);
+#pragma unroll
+        for (int i = 0; i < TM && is_a; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) load_a(rsa, a_off, i, h, d);
+    };
+    auto stage_b = [&](int d, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < PB; ++t) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) split_b(t, e, d);
+#pragma unroll
+            for (int p = 0; p < NB; ++p) write_b(t, p, stage);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        load_set(false, d, d * BK);
+        load_set(true, d, d * BK);
+    }
+    stage_b(0, 0);
+    load_set(false, 0, D * BK);
+#pragma unroll
+    for (int i = 0; i < 4 * TM; ++i) split_a(i / 4, i % 4, 0, 0);
+    load_set(true, 0, D * BK);
+    stage_b(1 % D, kStage);
+    load_set(false, 1 % D, (1 + D) * BK);
+    barrier();
+#pragma unroll
+    for (int p = 0; p < NB; ++p) read_b(p, 0, 0);
+    int s0 = 0, s1 = kStage, s2 = 2 * kStage;  // the stages of slices kt, kt + 1, kt + 2
+    for (int kt0 = 0; kt0 < nk; kt0 += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kt = kt0 + u;
+            slice(u & 1, (u + 1) & 1, s0, s1, s2, (u + 2) % D, (kt + 2 + D) * BK, (u + 1) % D, (kt + 1 + D) * BK);
+            barrier();
+            const int s = s0;
+            s0 = s1;
+            s1 = s2;
+            s2 = s;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += cor[i][j];
+
+    // ---- epilogue.  The tile's sums go through LDS (free: the loop's last
+    // barrier follows every wave's last read) and are written as whole 16-byte
+    // pieces of C rows, consecutive lanes a row's consecutive pieces.  Lane
+    // (c, g) holds rows 4 g + e, column c of each MFMA tile; with two wave
+    // groups, group 1 adds its half of the k first.  The code is kept short --
+    // one loop per activation, the recomputation rolled and apart -- because a
+    // launch runs it once, from a cold instruction cache: unrolled with every
+    // activation in every element it cost 36 k cycles a tile (16 of the 102 us of
+    // 1500x5120x1280).
+    float *const ct = (float *)lds;
+    int suspect = 0;
+    auto put = [&](bool add) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float *const to = &ct[(wm0 + 16 * i + 4 * g + e) * CS + wn0 + 16 * j + c];
+                    const float v = add ? *to + acc[i][j][e] : acc[i][j][e];
+                    suspect |= sbf_suspect(v);
+                    *to = v;
+                }
+    };
+    if constexpr (KW == 1) {
+        put(false);
+    } else {
+        if (kg == 1) put(false);
+        suspect = 0;
+        __syncthreads();
+        if (kg == 0) put(true);
+    }
+    if (__syncthreads_or(suspect)) {
+#pragma unroll 1
+        for (int e = tid; e < BM * BN; e += NT) {
+            const int tr = e / BN, row = m0 + tr, col = n0 + e % BN;
+            float *const v = &ct[tr * CS + e % BN];
+            if (row < a.M && col < a.N && sbf_suspect(*v)) *v = sbf_fp32_sum<FMT>(a, row, col);
+        }
+        __syncthreads();
+    }
+    constexpr int CH = BN / 4, RPP = NT / CH;  // 16-byte pieces of a tile row; rows a pass
+    const int pc = 4 * (tid % CH), tr0 = tid / CH, col = n0 + pc;  // a thread's pieces lie in one column of pieces
+    if (tr0 >= RPP || col >= a.N) return;
+    const int tr_end = min(BM, a.M - m0);
+    auto scalar_piece = [&](int tr) {
+        const size_t o = (size_t)(m0 + tr) * a.N + col;
+#pragma unroll 1
+        for (int q = 0; q < 4 && col + q < a.N; ++q) {
+            float v = a.alpha * ct[tr * CS + pc + q];
+            if (a.beta != 0.0f) v += a.beta * a.C[o + q];
+            if (a.bias) v += a.bias[col + q];
+            if (a.res) v += a.res[o + q];
+            tml_store_c(a.C + o + q, tml_apply_act(v, a.act, (long long)o + q, a.tail0));
+        }
+    };
+    // UN rows' loads in flight together
+    auto finish = [&](auto act_tag, auto un_tag) __attribute__((always_inline)) {
+        constexpr int ACT = decltype(act_tag)::value, UN = decltype(un_tag)::value;
+        floatx4 bias4 = {0.f, 0.f, 0.f, 0.f};
+        if (a.bias) bias4 = *(const floatx4 *)(a.bias + col);
+#pragma unroll 1
+        for (int tr = tr0; tr < tr_end; tr += UN * RPP) {
+            floatx4 v4[UN], cv[UN], rv[UN];
+#pragma unroll
+            for (int p = 0; p < UN; ++p) {
+                const int t = min(tr + p * RPP, tr_end - 1);
+                const size_t o = (size_t)(m0 + t) * a.N + col;
+                v4[p] = *(const floatx4 *)&ct[t * CS + pc];
+                if (a.beta != 0.0f) cv[p] = *(const floatx4 *)(a.C + o);
+                if (a.res) rv[p] = *(const floatx4 *)(a.res + o);
+            }
+#pragma unroll
+            for (int p = 0; p < UN; ++p) {
+                const int t = tr + p * RPP;
+                if (t >= tr_end) break;
+                const size_t o = (size_t)(m0 + t) * a.N + col;
+                if (ACT == TML_ACT_GELU_TANH && (long long)o + 4 > a.tail0) {  // the exact tanh of the flat tail
+                    scalar_piece(t);
+                    continue;
+                }
+                floatx4 out;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float v = a.alpha * v4[p][q];
+                    if (a.beta != 0.0f) v += a.beta * cv[p][q];
+                    if (a.bias) v += bias4[q];
+                    if (a.res) v += rv[p][q];
+                    out[q] = tml_apply_act(v, ACT, 0, 1);
+                }
+                tml_store_c(a.C + o, out);
+            }
+        }
+    };
+    using un4 = std::integral_constant<int, 4>;
+    using un2 = std::integral_constant<int, 2>;
+    if (!a.vec_epi) {
+#pragma unroll 1
+        for (int tr = tr0; tr < tr_end; tr += RPP) scalar_piece(tr);
+    } else if (a.act == TML_ACT_GELU_ERF) {
+        finish(std::integral_constant<int, TML_ACT_GELU_ERF>{}, un2{});
+    } else if (a.act == TML_ACT_GELU_TANH) {
+        finish(std::integral_constant<int, TML_ACT_GELU_TANH>{}, un2{});
+    } else {
+        finish(std::integral_constant<int, TML_ACT_NONE>{}, un4{});
+    }
+}
+
+// Tile configs (index = TML_GEMM_SBF_TILE - 1) and the terms of pick_sbf's
+// model: a launch with one tile a CU at most takes fixed + slices * (one +
+// busy * the share of busy CUs past 0.4), a slice being bk deep.
+struct SbfCfg {
+    int bm, bn, bk;
+    double fixed, one, busy;
+    double f16, q8k;  // the slice's cost in these formats, relative to f32 (0: not used)
+};
+constexpr SbfCfg kSbfCfgs[] = {
+    {256, 128, 32, 9.7, 1.58, 1.25, 0.86, 0.0},  // eight waves of 32 x 128
+    {256, 96, 32, 8.9, 1.33, 0.95, 0.86, 1.05},  // eight waves of 32 x 96
+    {128, 64, 64, 8.2, 1.13, 0.37, 0.91, 1.09},  // two wave groups of four 32 x 64
+    {128, 64, 32, 6.4, 0.67, 0.13, 0.86, 1.12},  // four waves of 32 x 64, two workgroups a CU
+    {64, 64, 32, 5.1, 0.49, 0.03, 0.83, 1.22},   // four waves of 16 x 64, three workgroups a CU
+};
+constexpr int kSbfNumCfgs = (int)(sizeof(kSbfCfgs) / sizeof(kSbfCfgs[0]));
+
+template <int FMT>
+void launch_sbf_cfg(int cfg, unsigned grid, const SbfArgs &a, hipStream_t s) {
+    switch (cfg) {
+        case 0: gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
+        case 1: gemm_sbf_kernel<FMT, 256, 96, 32, 96, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
+        case 2: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 64, 2, 8, 2><<<grid, 512, 0, s>>>(a); break;
+        case 3: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
+        default: gemm_sbf_kernel<FMT, 64, 64, 16, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
+    }
+}
+
+}  // namespace
+
+bool gemm_sbf_supported(const MatmulArgs &m) {
+    if (m.fmt != TML_FMT_F32 && m.fmt != TML_FMT_F16 && m.fmt != TML_FMT_Q8_K) return false;
+    if (m.M <= kGemvMaxM || m.K <= 0 || m.K % 4 != 0 || ((uintptr_t)m.A % 16) != 0) return false;
+    const uint64_t esz = m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1;
+    if ((uintptr_t)m.B % esz != 0) return false;
+    if (m.fmt == TML_FMT_Q8_K && (m.block != 32 || m.N % 32 != 0 || ((uintptr_t)m.scales % 4) != 0)) return false;
+    if (env_int("TML_GEMM_SBF", 1) == 0) return false;
+    // every buffer offset below 2^31: A rows up to M + 256, B k-rows up to K + 512
+    const uint64_t lim = (uint64_t)1 << 31;
+    return (uint64_t)(m.M + 256) * (uint64_t)m.K * 4u < lim && (uint64_t)(m.K + 512) * (uint64_t)m.N * esz < lim &&
+           m.M < ((int64_t)1 << 30) && m.N < ((int64_t)1 << 30);
+}
+
+// The tile of least modelled time, if that is below `other_us`, the modelled
+// time of the fp32-MFMA kernels' plan (0.97 of it for f32, whose model is the
+// older one).  The terms were fitted to a sweep of the five tiles on MI355X over
+// M = 200-2048 and N, K = 384-5120 in the three formats (22 shapes; every launch
+// reading one of 8 weight copies).  Measured, us, fp32 MFMA / this kernel's pick:
+//   f32  1500x3840x1280 137 / 80 (256x96), 1500x5120x1280 165 / 95 (256x128),
+//        1500x1280x5120 162 / 115 and 1500x1280x1280 51 / 33 (128x64x64),
+//        512x4096x1024 40.0 / 29.5, 1024x3072x768 47.1 / 35.3 (64x64),
+//        2048x768x3072 83 / 69; where it loses and stays unpicked: 512x1024x1024
+//        13.7 / 21, 512x384x384 5.1 / 10.5, 512x1024x4096 42.8 / 69 (few tiles),
+//        256x3072x1024 18.5 / 21;
+//   F16  1500x3840x1280 140 / 69, 1500x1280x5120 169 / 105, 512x4096x1024 40.1 /
+//        27.1, 1500x1536x384 19.7 / 17.8, 391x1536x384 11.2 / 9.8;
+//   Q8_K 1500x3840x1280 159 / 82, 1500x1280x5120 185 / 127, 512x4096x1024 44.7 /
+//        31.9, 1024x3072x768 50.2 / 39.7.
+// 2-norm error against 64 bits, the same shapes: 3.7e-7 - 9.9e-7 / 0.9e-7 - 4.5e-7.
+bool pick_sbf(const MatmulArgs &m, double other_us, GemmPlan *p) {
+    constexpr double kCus = 256.0;
+    double best = other_us * (m.fmt == TML_FMT_F32 ? 0.97 : 1.0);
+    int cfg = -1;
+    for (int c = 0; c < kSbfNumCfgs; ++c) {
+        const SbfCfg &t = kSbfCfgs[c];
+        const double rel = m.fmt == TML_FMT_F32 ? 1.0 : m.fmt == TML_FMT_F16 ? t.f16 : t.q8k;
+        if (rel == 0.0) continue;
+        const double w = (double)(((m.M + t.bm - 1) / t.bm) * ((m.N + t.bn - 1) / t.bn)) / kCus;  // tiles a CU
+        const double busy = std::max(0.0, std::min(w, 1.0) - 0.4) * t.busy;
+        double us = t.fixed, slice = t.one + busy;  // one tile a CU
+        if (w > 1.0 && c < 3) {         // one workgroup a CU: whole rounds, each with its own fill and end
+            us += 4.0 * (std::ceil(w) - 1.0);
+            slice *= std::ceil(w);
+        } else if (w > 1.0 && c == 3) {  // two share a CU
+            slice = w <= 2.0 ? 1.25 + 0.2 * (w - 1.0) : 0.75 * w + 0.03;
+        } else if (w > 1.0) {            // three share a CU
+            slice = w <= 2.0 ? 0.69 + 0.16 * (w - 1.0) : w <= 3.0 ? 1.17 + 0.09 * (w - 2.0) : 0.44 * w + 0.02;
+        }
+        us += slice * rel * (double)((m.K + t.bk - 1) / t.bk);
+        if (us < best) {
+            best = us;
+            cfg = c;
+        }
+    }
+    const int forced = env_int("TML_GEMM_SBF_TILE", 0) - 1;
+    if (forced >= 0 && forced < kSbfNumCfgs) cfg = forced;
+    if (cfg < 0) return false;
+    p->cfg = cfg;
+    p->nsplit = 1;
+    p->tiles = (int)(((m.M + kSbfCfgs[cfg].bm - 1) / kSbfCfgs[cfg].bm) * ((m.N + kSbfCfgs[cfg].bn - 1) / kSbfCfgs[cfg].bn));
+    return true;
+}
+
+Status launch_gemm_sbf(const MatmulArgs &m, const GemmPlan &p, hipStream_t s) {
+    if (!gemm_sbf_supported(m) || p.cfg < 0 || p.cfg >= kSbfNumCfgs)
+        return Status::Err(TML_ERR_INVALID_ARG, "split-bf16 GEMM: operands or tile config not supported");
+    SbfArgs a;
+    a.M = (int)m.M; a.N = (int)m.N; a.K = (int)m.K;
+    a.A = m.A; a.B = (const uint8_t *)m.B; a.scales = m.scales;
+    a.ldb = (int)(m.N * (m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1));
+    a.bias = m.bias; a.res = m.res; a.C = m.C;
+    a.alpha = m.alpha_eff; a.beta = m.beta;
+    a.act = m.act;
+    a.tail0 = tml_act_tail0((long long)m.M * m.N);
+    a.a_bytes = (unsigned)((uint64_t)m.M * (uint64_t)m.K * 4u);
+    a.b_bytes = (unsigned)((uint64_t)m.K * (uint64_t)a.ldb);
+    a.s_bytes = m.fmt == TML_FMT_Q8_K ? (unsigned)((uint64_t)m.K * (uint64_t)m.N / 32u * 4u) : 0u;
+    a.tiles_m = (int)((m.M + kSbfCfgs[p.cfg].bm - 1) / kSbfCfgs[p.cfg].bm);
+    a.tiles_n = (int)((m.N + kSbfCfgs[p.cfg].bn - 1) / kSbfCfgs[p.cfg].bn);
+    a.vec_epi = m.N % 4 == 0 && ((uintptr_t)m.C % 16) == 0 && (m.bias == nullptr || ((uintptr_t)m.bias % 16) == 0) &&
+                (m.res == nullptr || ((uintptr_t)m.res % 16) == 0);
+    const int64_t grid = (int64_t)a.tiles_m * a.tiles_n;
+    if (grid >= ((int64_t)1 << 31)) return Status::Err(TML_ERR_INVALID_SHAPE, "split-bf16 GEMM: grid too large");
+    switch (m.fmt) {
+        case TML_FMT_F32: launch_sbf_cfg<TML_FMT_F32>(p.cfg, (unsigned)grid, a, s); break;
+        case TML_FMT_F16: launch_sbf_cfg<TML_FMT_F16>(p.cfg, (unsigned)grid, a, s); break;
+        default: launch_sbf_cfg<TML_FMT_Q8_K>(p.cfg, (unsigned)grid, a, s); break;
+    }
+    TML_HIP_TRY(hipGetLastError());
+    return Status::Ok();
+}
+
+}  // namespace tml

@@ -185,6 +185,7 @@ struct GemmPlan {
     int spl = 0;       // BK-slices per split
     int tiles = 0;
     bool fused = false;  // split-K partials combined in the GEMM kernel (no reduce launch)
+    bool sbf = false;    // f32 / F16 / Q8_K on the bf16 matrix cores (gemm_sbf.hip; cfg its tile)
     bool qbf = false;    // Q8_0 / Q4_0 on the bf16 matrix cores (gemm_qbf.hip; cfg, nsplit, spl its plan)
 };
 GemmPlan plan_gemm(const MatmulArgs &a);
@@ -205,6 +206,12 @@ Status launch_gemm_f32_dma(const MatmulArgs &a, const GemmPlan &p, const Workspa
 bool gemm_qbf_supported(const MatmulArgs &a);
 void pick_qbf(const MatmulArgs &a, GemmPlan *p);
 Status launch_gemm_qbf(const MatmulArgs &a, const GemmPlan &p, const Workspace &ws, hipStream_t s);
+// f32 / F16 / Q8_K GEMM on the bf16 matrix cores (gemm_sbf.hip): M >
+// kGemvMaxM, K % 4 == 0, 16-byte aligned A.  pick_sbf is false where the
+// fp32-MFMA kernels, at a modelled other_us, are the faster choice.
+bool gemm_sbf_supported(const MatmulArgs &a);
+bool pick_sbf(const MatmulArgs &a, double other_us, GemmPlan *p);
+Status launch_gemm_sbf(const MatmulArgs &a, const GemmPlan &p, hipStream_t s);
 // C = act(alpha * sum of the nsplit [M,N] partials (in split order) * colscale + beta * C + bias + res).
 Status launch_splitk_reduce(const float *partials, int nsplit, const MatmulArgs &a, hipStream_t s);
 void gemm_dma_workspace_need(const MatmulArgs &a, const GemmPlan &p, size_t *partial_floats, size_t *counters);
