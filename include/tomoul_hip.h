@@ -237,7 +237,8 @@ int tml_hip_weight_release(const void *host);
  * split-K workspace, which the library grows (hipMalloc) the first time a
  * call needs more than earlier calls did.  Growth is refused with
  * TML_ERR_INVALID_ARG while `stream` is being captured, so run every call
- * once eagerly before capturing it.  A grown workspace never frees the old
+ * once eagerly before capturing it.  (Where only the split-bf16 kernel's K
+ * split asks for the growth, a captured call runs an unsplit plan instead.)  A grown workspace never frees the old
  * one before tml_hip_shutdown: a graph captured earlier stays valid however
  * the workspace grows afterwards. */
 int tml_hip_gemm_dev(int fmt, int64_t M, int64_t N, int64_t K, const float *A, const void *B, float scale,

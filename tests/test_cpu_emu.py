@@ -328,9 +328,9 @@ def test_noalloc_entry_point(emu):
 
 
 def test_sbf_cases(emu):
-    # the split-bf16 GEMM (TML_GEMM_SBF_TILE 1-5): every tile and format on shapes
-    # ragged in M, N and K, odd N, the smallest K, every epilogue; the planner's
-    # own choice at encoder sizes; and a short operand, which must be reported
+    # the split-bf16 GEMM (TML_GEMM_SBF_TILE 1-5, int8 / int4 1-2): every tile and
+    # format on shapes ragged in M, N and K, odd N, the smallest K, every epilogue,
+    # K splits; the planner's own choice at encoder sizes; and a short operand, which must be reported
     cases = []
     for tile in range(1, 6):
         env = f"TML_GEMM_SBF_TILE={tile}"
@@ -339,6 +339,15 @@ def test_sbf_cases(emu):
                             (Q8_K, [(200, 352, 516), (33, 128, 40), (300, 64, 1288)])]:
             for (M, N, K) in shapes:
                 cases += [f"gemm {fmt} {M} {N} {K} br {env}", f"gemm {fmt} {M} {N} {K} teB {env}"]
+    for fmt in (Q8_0, Q4_0, Q8_0_PC, Q4_0_PC):
+        for tile in (1, 2):
+            for split in (1, 3):
+                env = f"TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT={split}"
+                cases += [f"gemm {fmt} {M} {N} {K} br {env}" for (M, N, K) in [(200, 328, 520), (33, 130, 40),
+                                                                              (300, 70, 1288), (257, 514, 36)]]
+    for tile in range(1, 6):
+        cases += [f"gemm 0 130 97 516 br TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT=3",
+                  f"noalloc 3 257 192 260 b TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT=2"]
     cases += ["gemm 0 1500 3840 64 b", "gemm 4 1500 3840 64 e", "gemm 3 1500 3840 64 br", "gemm 0 100 1001 388 bt"]
     outs, fails = run_cases(emu, cases)
     assert not fails and not _err_lines(outs), (fails, _err_lines(outs)[:3])

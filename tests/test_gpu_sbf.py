@@ -1,4 +1,4 @@
-"""The split-bf16 GEMM (gemm_sbf.hip: f32 / F16 / Q8_K weights, M > 8) against 64-bit products.
+"""The split-bf16 GEMM (gemm_sbf.hip, M > 8, every weight format) against 64-bit products.
 
 Every operand is split exactly into bf16 terms and the products of the terms
 that matter are summed in fp32, so an output differs from the 64-bit product
@@ -9,7 +9,11 @@ the epilogue's own roundings:
 Operands the split does not carry (infinities, NaNs, values past the largest
 bf16, sums of products below 2^-70) are recomputed in fp32 in ascending k, as
 the reference does (src/core/ops.zig:277-414), so their inf / NaN pattern is the
-oracle's.  TML_GEMM_SBF_TILE picks a tile, TML_GEMM_SBF=0 turns the kernel off.
+oracle's.  Int8 / int4 weights take two terms of A (|x - hi - lo| <= 2^-17 |x|) and
+share one sum, which a slice rounds twice:
+    |C - ref| <= (2^-17 + (2 ceil(K / 32) + 8) * 2^-24) * sum_k |a b| + 2^-23 |ref|.
+A K split adds one rounding a split.  TML_GEMM_SBF_TILE / _SPLIT pick a tile and
+a K split, TML_GEMM_SBF=0 turns the kernel off.
 """
 import os
 
@@ -24,7 +28,7 @@ TILES = (1, 2, 3, 4, 5)
 
 @pytest.fixture
 def env():
-    keys = ("TML_GEMM_SBF_TILE", "TML_GEMM_SBF")
+    keys = ("TML_GEMM_SBF_TILE", "TML_GEMM_SBF_SPLIT", "TML_GEMM_SBF", "TML_REQUIRE_SPLIT")
     saved = {key: os.environ.get(key) for key in keys}
     yield os.environ
     for key, v in saved.items():
@@ -52,10 +56,11 @@ def run(fmt, m, n, k, a, q, scales, **kw):
     return c
 
 
-def check(c, a, w, bias=None, res=None):
+def check(c, a, w, bias=None, res=None, terms=3):
     ref = a.astype(np.float64) @ w.astype(np.float64)
     mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64)
-    bound = (-(-a.shape[1] // 32) + 8) * 2.0**-24 * mag
+    slices = -(-a.shape[1] // 32)
+    bound = ((slices + 8) * 2.0**-24 if terms == 3 else 2.0**-17 + (2 * slices + 8) * 2.0**-24) * mag
     for x in (bias, res):
         if x is not None:
             ref = ref + x
@@ -131,3 +136,82 @@ def test_sbf_exact_integers(env):
     for tile in TILES:
         env["TML_GEMM_SBF_TILE"] = str(tile)
         assert np.array_equal(run(_abi.FMT_F32, 200, 129, 320, a, w, None), a @ w)
+
+
+@pytest.mark.parametrize("split", [2, 3])
+@pytest.mark.parametrize("tile", TILES)
+def test_sbf_split(env, tile, split):
+    # raw partials of K splits (the last one short), added in split order by the
+    # reduce launch with bias and residual; odd N takes the scalar partial stores
+    env["TML_GEMM_SBF_TILE"], env["TML_GEMM_SBF_SPLIT"], env["TML_REQUIRE_SPLIT"] = str(tile), str(split), "1"
+    for (m, n, k) in [(130, 97, 516), (257, 200, 260)]:
+        a, bias, res = synth.normal_matrix(51, m, k), synth.normal(52, n, 0.0, 0.02), synth.normal_matrix(53, m, n)
+        w = synth.normal_matrix(54, k, n, 0.02)
+        c = np.zeros((m, n), np.float32)
+        _abi.gemm_residual(_abi.FMT_F32, m, n, k, a, w, res, c, bias=bias)
+        check(c, a, w, bias.astype(np.float64), res.astype(np.float64))
+
+
+@pytest.mark.parametrize("tile,split", [(1, 1), (1, 3), (2, 1), (2, 2)])
+def test_sbf_int(orc, env, tile, split):
+    env["TML_GEMM_SBF_TILE"], env["TML_GEMM_SBF_SPLIT"] = str(tile), str(split)
+    for (m, n, k) in [(9, 34, 40), (300, 130, 520), (257, 98, 1288)]:
+        a, bias = synth.normal_matrix(61 + m, m, k), synth.normal(62, n, 0.0, 0.02)
+        w = synth.normal_matrix(63, k, n, 0.02)
+        q, s = orc.quantize_q8(w)
+        p, s4 = orc.quantize_q4(w)
+        qc, sc = orc.quantize_q8_cols(w)
+        pc, sc4 = orc.quantize_q4_cols(w)
+        for fmt, b, scale, scales, deq in [
+                (_abi.FMT_Q8_0, q, s, None, orc.dequantize_q8(q, s)),
+                (_abi.FMT_Q4_0, p, s4, None, orc.dequantize_q4(p, k * n, s4)),
+                (_abi.FMT_Q8_0_PC, qc, 1.0, sc, orc.dequantize_cols(_abi.FMT_Q8_0_PC, qc, sc, k, n)),
+                (_abi.FMT_Q4_0_PC, pc, 1.0, sc4, orc.dequantize_cols(_abi.FMT_Q4_0_PC, pc, sc4, k, n))]:
+            c = run(fmt, m, n, k, a, b, scales, scale=scale, bias=bias)
+            check(c, a, np.asarray(deq, np.float32).reshape(k, n), bias.astype(np.float64), terms=2)
+
+
+@pytest.mark.parametrize("tile", [1, 2])
+def test_sbf_int_inf_nan(orc, env, tile):
+    env["TML_GEMM_SBF_TILE"] = str(tile)
+    m, n, k = 140, 100, 72
+    a = synth.normal_matrix(71, m, k)
+    a[3, 5], a[4, 0], a[64, 71], a[139, 7] = np.inf, -np.inf, np.nan, np.float32(3.4028235e38)
+    q, s = orc.quantize_q8(synth.normal_matrix(72, k, n, 0.02))
+    q = q.reshape(k, n).copy()
+    q[7] = np.clip(q[7], -1, 1)  # FLT_MAX times these stays finite
+    q[5, ::7] = 0
+    c, ref = run(_abi.FMT_Q8_0, m, n, k, a, q, None, scale=s), orc.matmul_q8(a, q, s)
+    assert np.array_equal(np.isnan(c), np.isnan(ref)) and np.array_equal(np.isinf(c), np.isinf(ref))
+    fin = np.isfinite(ref)
+    mag = np.where(np.isfinite(a), np.abs(a), 0).astype(np.float64) @ np.abs(q.astype(np.float64) * s)
+    assert np.all(np.abs(c[fin].astype(np.float64) - ref[fin]) <= (2.0**-17 + 2.0**-23 * k) * mag[fin])
+
+
+def test_sbf_split_plan_without_workspace(env):
+    """512 x 1024 x 4096 in f32 splits K by default; a first call under stream
+    capture, where the workspace cannot grow, runs an unsplit plan instead of
+    being refused, and the allocation-free call serves the split one."""
+    import torch
+    torch.cuda.synchronize()
+    _abi.shutdown()  # a fresh context has no workspace
+    _abi.init()
+    m, n, k = 512, 1024, 4096
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    a, b = torch.randn(m, k, generator=gen, device="cuda"), torch.randn(k, n, generator=gen, device="cuda") * 0.02
+    c = [torch.zeros(m, n, device="cuda") for _ in range(3)]
+    ref = (a.double() @ b.double())
+    side, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=side):
+        _abi.gemm_dev(_abi.FMT_F32, m, n, k, a.data_ptr(), b.data_ptr(), c[0].data_ptr(), stream=side.cuda_stream)
+    env["TML_REQUIRE_SPLIT"] = "1"
+    _abi.gemm_ex_dev_noalloc(_abi.FMT_F32, m, n, k, a.data_ptr(), b.data_ptr(), c[1].data_ptr())
+    _abi.gemm_dev(_abi.FMT_F32, m, n, k, a.data_ptr(), b.data_ptr(), c[2].data_ptr())
+    for _ in range(3):
+        c[0].zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        for x in c:
+            assert float((x - ref).norm() / ref.norm()) <= 2e-6
+    assert torch.equal(c[1], c[2])

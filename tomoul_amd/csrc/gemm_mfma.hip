@@ -655,8 +655,16 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
     const bool fp32_forced = set("TML_GEMM_DMA_Q") || set("TML_GEMM_TILE") || set("TML_GEMM_DMA_TILE") ||
                              set("TML_GEMM_SPLIT");
     if (!fp32_forced && gemm_qbf_supported(m)) {
+        // ... or, at the largest sizes (where pick_qbf models its time), the
+        // split-bf16 kernel if that is modelled faster
         p.qbf = true;
-        pick_qbf(m, &p);
+        const double qbf_us = pick_qbf(m, &p);
+        const bool qbf_forced = set("TML_GEMM_QBF") || set("TML_GEMM_QBF_TILE") || set("TML_GEMM_QBF_SPLIT");
+        GemmPlan q;
+        if (!qbf_forced && gemm_sbf_supported(m) && pick_sbf(m, qbf_us, p.nsplit, &q)) {
+            q.sbf = true;
+            return q;
+        }
         return p;
     }
     // f32 B takes the direct-copy kernel whenever its rows allow it.  For
@@ -713,7 +721,8 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
     const bool other_forced = fp32_forced || set("TML_GEMM_DMA") || set("TML_GEMM_FUSED") || set("TML_GEMM_XCDPART") ||
                               set("TML_GEMM_XCD") || set("TML_GEMM_GROUPM");
     GemmPlan q;
-    if (!other_forced && gemm_sbf_supported(m) && pick_sbf(m, other_us, &q)) {
+    if (!other_forced && m.fmt != TML_FMT_Q8_0 && m.fmt != TML_FMT_Q4_0 && gemm_sbf_supported(m) &&
+        pick_sbf(m, other_us, p.nsplit, &q)) {
         q.sbf = true;
         return q;
     }
@@ -724,7 +733,7 @@ void gemm_workspace_need(const MatmulArgs &m, size_t *partial_floats, size_t *co
     const GemmPlan p = plan_gemm(m);
     *partial_floats = 0;
     *counters = 0;
-    if (p.qbf && p.nsplit > 1) *partial_floats = (size_t)p.nsplit * (size_t)m.M * (size_t)m.N;
+    if ((p.qbf || p.sbf) && p.nsplit > 1) *partial_floats = (size_t)p.nsplit * (size_t)m.M * (size_t)m.N;
     if (p.dma && p.nsplit > 1) gemm_dma_workspace_need(m, p, partial_floats, counters);
 }
 
@@ -767,9 +776,9 @@ Status launch_gemm_mfma(const MatmulArgs &m, const Workspace &ws, hipStream_t s)
                            "the largest size the tests run them at");
     const GemmPlan p = plan_gemm(m);
     // TML_REQUIRE_SPLIT=1 (tests): refuse a plan that does not split K
-    if (!((p.qbf || p.dma) && p.nsplit > 1) && env_int("TML_REQUIRE_SPLIT", 0) == 1)
+    if (!((p.qbf || p.dma || p.sbf) && p.nsplit > 1) && env_int("TML_REQUIRE_SPLIT", 0) == 1)
         return Status::Err(TML_ERR_INVALID_ARG, "TML_REQUIRE_SPLIT=1: this call's plan does not split K");
-    if (p.sbf) return launch_gemm_sbf(m, p, s);
+    if (p.sbf) return launch_gemm_sbf(m, p, ws, s);
     if (p.qbf) return launch_gemm_qbf(m, p, ws, s);
     if (p.dma) return launch_gemm_f32_dma(m, p, ws, s);
     const int cus = device_cus();

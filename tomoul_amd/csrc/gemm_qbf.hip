@@ -556,7 +556,7 @@ void launch_qbf_cfg(int cfg, unsigned grid, const QbfArgs &a, hipStream_t s) {
 //     bytes, competes with the main loop): 128 x 128 at s = 2 measured
 //     53.1 us at 1500x3840x1280, 67.6 at 1500x5120x1280 and 35.0 at
 //     1024x4096x1024, 9-13 us above the model.
-void pick_qbf(const MatmulArgs &m, GemmPlan *p) {
+double pick_qbf(const MatmulArgs &m, GemmPlan *p) {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
         int n = 0;
@@ -571,6 +571,7 @@ void pick_qbf(const MatmulArgs &m, GemmPlan *p) {
     };
     int cfg = 8;
     int64_t nsplit = 1;
+    double modelled_us = 0.0;
     // the modelled time of config c at s splits (the plan's own rounding of
     // the slices into whole BK-deep ones per split)
     auto modelled = [&](int c, int64_t ns, double c_one, double c_many, double per_split, double traffic) {
@@ -628,6 +629,7 @@ void pick_qbf(const MatmulArgs &m, GemmPlan *p) {
                     nsplit = ns;
                 }
             }
+        modelled_us = best;
     }
     if (cfg == 7) {
         // Four 64-deep slices of loads in flight instead of two (config 10)
@@ -653,6 +655,7 @@ void pick_qbf(const MatmulArgs &m, GemmPlan *p) {
     p->nsplit = (int)nsplit;
     p->spl = (int)std::max<int64_t>(spl, 1);
     p->tiles = (int)tiles_of(cfg);
+    return modelled_us;
 }
 
 bool gemm_qbf_supported(const MatmulArgs &m) {

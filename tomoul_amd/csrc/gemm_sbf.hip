@@ -1,5 +1,6 @@
-// gemm_sbf.hip -- f32 / F16 / Q8_K GEMM on the bf16 matrix cores, every
-// operand split exactly into bf16 terms.
+// gemm_sbf.hip -- GEMM on the bf16 matrix cores, fp32 values split into bf16
+// terms: f32, F16 and Q8_K weights (both operands exactly), and the largest int8 /
+// int4 ones (A in two terms, as in gemm_qbf.hip).
 //
 //   C[M,N] = act(alpha * A[M,K] . B[K,N] + beta * C + bias[N] + R)
 //
@@ -17,11 +18,15 @@
 // once where the fp32 matrix cores round theirs eight times: the 2-norm error
 // against 64 bits is 0.9e-7 - 4.5e-7 over the shapes at pick_sbf, theirs 3.7e-7 -
 // 9.9e-7.
+// Int8 and int4 weights are exact in bf16 and A takes two terms, |x - hi - lo| <=
+// 2^-17 |x|: two products, the arithmetic of gemm_qbf.hip.
 //
 // Bound: the matrix cores, at the clock the power limit leaves them.  At
 // 1500x5120x1280 (240 tiles of 256x128) the main loop keeps them 82 % busy, at
 // 1.85 GHz (2.3 GHz with 48 CUs busy): 95 us, 207 TFLOP/s, 165 us before on the
-// fp32 matrix cores.
+// fp32 matrix cores.  Int8, same shape: 49 us, 401 TFLOP/s of algorithmic work; its
+// two products take a third of the matrix-core time, and LDS and the loads' issue
+// are as large.
 //
 // Values the split does not carry -- infinities and NaNs (their residual is
 // NaN), |x| above the largest bf16, and magnitudes so small that l falls under
@@ -48,18 +53,21 @@ constexpr int kSbfXcd = 8;  // XCDs of an MI355X: workgroups are dealt to them r
 struct SbfArgs {
     int M, N, K;
     const float *A;         // [M,K], K % 4 == 0, 16-byte aligned
-    const uint8_t *B;       // [K,N]: f32, binary16 or int8
+    const uint8_t *B;       // [K,N]: f32, binary16, int8, or int4 two a byte (even n in the low nibble)
     const float *scales;    // Q8_K block scales (32 elements each, N % 32 == 0)
     int ldb;                // bytes per B row
+    const float *colscale;  // [N] per-column factor on A.B, or nullptr
     const float *bias;      // [N] or nullptr
     const float *res;       // [M,N] residual after the bias, or nullptr (may equal C)
     float *C;
     float alpha, beta;
     int act;
     long long tail0;
-    unsigned a_bytes, b_bytes, s_bytes;  // M * K * 4, K * ldb, scale bytes
+    unsigned a_bytes, s_bytes;  // M * K * 4, scale bytes
     int tiles_m, tiles_n;
-    int vec_epi;            // N % 4 == 0 and C, bias, residual 16-byte aligned
+    int nsplit, spl;        // K splits, k a split (a multiple of the slice)
+    float *ws;              // nsplit > 1: [nsplit][M][N] raw partials
+    int vec_epi;            // N % 4 == 0 and C, bias, residual, column scales 16-byte aligned
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t sbf_rsrc(const void *base, unsigned nbytes) {
@@ -94,15 +102,27 @@ __device__ __forceinline__ int sbf_slot(int r, int s) {
     else return r * 8 + (s ^ (r & 7));
 }
 
-// bf16 terms of B: a binary16 weight is two exactly.
+// bf16 terms of A and B, and the pairs of them multiplied.
 template <int FMT>
-constexpr int kSbfPlanesB = FMT == TML_FMT_F16 ? 2 : 3;
+constexpr bool kSbfInt = FMT == TML_FMT_Q8_0 || FMT == TML_FMT_Q4_0;
+template <int FMT>
+constexpr int kSbfPlanesA = kSbfInt<FMT> ? 2 : 3;
+template <int FMT>
+constexpr int kSbfPlanesB = kSbfInt<FMT> ? 1 : FMT == TML_FMT_F16 ? 2 : 3;
+template <int FMT>
+constexpr int kSbfProducts = kSbfInt<FMT> ? 2 : FMT == TML_FMT_F16 ? 5 : 6;
+// The int4 value of column n in the byte that holds it.
+__device__ __forceinline__ float sbf_int4(uint32_t byte, int n) {
+    return (float)((int32_t)(byte << ((n & 1) ? 24 : 28)) >> 28);
+}
 
 // One element of B as the f32 the reference multiplies by.
 template <int FMT>
 __device__ __forceinline__ float sbf_b(const SbfArgs &a, int k, int n) {
     if constexpr (FMT == TML_FMT_F32) return ((const float *)a.B)[(size_t)k * a.N + n];
     else if constexpr (FMT == TML_FMT_F16) return tml_half_bits(((const uint16_t *)a.B)[(size_t)k * a.N + n]);
+    else if constexpr (FMT == TML_FMT_Q8_0) return (float)((const int8_t *)a.B)[(size_t)k * a.N + n];
+    else if constexpr (FMT == TML_FMT_Q4_0) return sbf_int4(a.B[(size_t)k * a.ldb + n / 2], n);
     else return (float)((const int8_t *)a.B)[(size_t)k * a.N + n] * a.scales[((size_t)k * a.N + n) >> 5];
 }
 
@@ -111,18 +131,22 @@ __device__ __forceinline__ bool sbf_suspect(float v) {
     const uint32_t u = __float_as_uint(v) & 0x7FFFFFFFu;
     return u - 1u >= 0x7F7FFFFFu || u - 1u < 0x1C7FFFFFu ? u != 0u : false;  // not finite, or 0 < |v| < 2^-70
 }
-// The ascending fp32 sum of output (row, col)'s products.
+// The ascending fp32 sum of output (row, col)'s products over k in [k0, k1).
 template <int FMT>
-__device__ __forceinline__ float sbf_fp32_sum(const SbfArgs &a, int row, int col) {
+__device__ __forceinline__ float sbf_fp32_sum(const SbfArgs &a, int row, int col, int k0, int k1) {
     float s = 0.0f;
-    for (int k = 0; k < a.K; ++k) s = fmaf(a.A[(size_t)row * a.K + k], sbf_b<FMT>(a, k, col), s);
+    for (int k = k0; k < k1; ++k) s = fmaf(a.A[(size_t)row * a.K + k], sbf_b<FMT>(a, k, col), s);
     return s;
 }
 
 // A workgroup of NW = 4 or 8 waves owns a BM x BN tile of C, each wave a WM x
 // WN sub-tile (or, with KW = 2 wave groups, half the k of one), and walks K in
 // BK-deep slices.  A wave loads the A it multiplies straight into registers, in
-// the MFMA's own layout, and splits it there; B is loaded once per workgroup,
+// the MFMA's own layout, and splits it there (int8 / int4, whose products are a
+// third: in whole 128-byte rows, turned through LDS rows of the wave's own -- a load
+// in the MFMA's layout takes 16 bytes of a row a lane, neighbouring lanes different
+// rows, and 30-40 cycles to issue; 1500x3840x1280 54.6 -> 45.3 us, while the
+// three-term formats, whose LDS is as busy as their matrix cores, lose up to 18 %); B is loaded once per workgroup,
 // split, and passed through three LDS stages as rows of 16-byte slots (8 k), one
 // barrier a slice: a slice is written two steps before it is multiplied, so its
 // first operands are read before the barrier that starts its step.  (With A in LDS too, its writes -- 64 bytes a clock -- and
@@ -140,7 +164,9 @@ template <int FMT, int BM, int BN, int WM, int WN, int BK, int KW, int NW, int D
 __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     static_assert(KW == 1 ? BK == 32 : KW == 2 && BK == 64, "each wave group multiplies one 32-k half of a slice");
     static_assert(NW == 4 || NW == 8, "one or two waves a SIMD");
-    constexpr int NA = 3, NB = kSbfPlanesB<FMT>;
+    constexpr int NA = kSbfPlanesA<FMT>, NB = kSbfPlanesB<FMT>, NP = kSbfProducts<FMT>;
+    constexpr bool AL = kSbfInt<FMT>;  // A through the waves' own LDS rows (below)
+    constexpr bool COR = NP > 2;  // the small products have accumulators of their own
     constexpr int SL = BK / 8;    // 16-byte slots (8 k) of an LDS row
     constexpr int NT = 64 * NW;
     constexpr int NWS = NW / KW;  // waves per group, one per sub-tile
@@ -152,7 +178,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 
     constexpr int kStage = BN * SL * NB;  // 16-byte slots of a stage
     constexpr int CS = BN + 4;            // floats of a staged C row (rows 4 apart: 16 banks on)
-    constexpr int kLds = 3 * kStage > BM * CS / 4 ? 3 * kStage : BM * CS / 4;
+    constexpr int kARows = 3 * kStage;    // AL: the waves' own A rows, WM x 8 slots each
+    constexpr int kLoop = kARows + (AL ? NW * WM * 8 : 0);
+    constexpr int kLds = kLoop > BM * CS / 4 ? kLoop : BM * CS / 4;
     __shared__ uintx4 lds[kLds];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -164,12 +192,15 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 
     // Workgroup -> tile: consecutive ids within each XCD (own L2), in groups
     // of eight tile rows so that neighbours share A rows and B columns.
-    int tile_m, tile_n;
+    // K splits split by split: an XCD's workgroups share one k range.
+    int tile_m, tile_n, split;
     {
         const int nblk = gridDim.x, b = blockIdx.x;
         const int per = nblk / kSbfXcd, rem = nblk % kSbfXcd;
         const int xcd = b % kSbfXcd, idx = b / kSbfXcd;
-        const int lin = (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+        int lin = (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+        split = lin / (a.tiles_m * a.tiles_n);
+        lin -= split * (a.tiles_m * a.tiles_n);
         constexpr int GM = 8;
         const int group = GM * a.tiles_n;
         const int first_m = (lin / group) * GM;
@@ -178,22 +209,28 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         tile_n = (lin % group) / gsize;
     }
     const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int kbase = split * a.spl, kend = min(a.K, kbase + a.spl);  // this split's k
 
     // ---- loads.  A lane's offsets are fixed; the slice moves the buffer's base
-    // and byte count (scalar work only).  Rows of A past M and k-rows of B past K
-    // lie past the byte count and read zeros.  A's k past K reads the next row,
+    // and byte count (scalar work only).  Rows of A past M and k-rows of B past
+    // kend lie past the byte count and read zeros.  A's k past kend reads on,
     // against B's zero rows; B columns past N read the next k-row and feed dropped
     // outputs.  (A value there that is not finite makes its sum a NaN, which the
     // epilogue recomputes.)
     constexpr unsigned ESZ = FMT == TML_FMT_F32 ? 4u : FMT == TML_FMT_F16 ? 2u : 1u;
-    const unsigned a_off = ((unsigned)c * (unsigned)a.K + 4u * (unsigned)g) * 4u;
+    auto col_bytes = [](unsigned n) constexpr { return FMT == TML_FMT_Q4_0 ? n / 2u : n * ESZ; };
+    const unsigned b_bytes = (unsigned)kend * (unsigned)a.ldb;
+    // A: AL loads 8 rows of 128 bytes an instruction (lane / 8, lane % 8), else 16
+    // rows' 16-byte pieces in the MFMA's layout (c, g)
+    const unsigned a_off = AL ? ((unsigned)(lane / 8) * (unsigned)a.K + 4u * (unsigned)(lane % 8)) * 4u
+                              : ((unsigned)c * (unsigned)a.K + 4u * (unsigned)g) * 4u;
     unsigned b_off[PB], s_off[PB];
     int slot_b[PB];
 #pragma unroll
     for (int t = 0; t < PB; ++t) {
         const int j = tid + t * NT, n = j % BN, sl = j / BN;
         const unsigned k = (unsigned)(32 * (sl / 4) + 4 * (sl % 4));
-        b_off[t] = k * (unsigned)a.ldb + (unsigned)n * ESZ;
+        b_off[t] = k * (unsigned)a.ldb + col_bytes((unsigned)n);
         s_off[t] = k * ((unsigned)a.N / 8u) + (unsigned)n / 32u * 4u;
         slot_b[t] = sbf_slot<SL>(n, sl % SL);
     }
@@ -203,13 +240,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     };
     // the buffers at a slice's first k
     auto at_a = [&](int k0) __attribute__((always_inline)) {
-        return moved(a.A, a.a_bytes, ((unsigned)(m0 + wm0) * (unsigned)a.K + (unsigned)(k0 + 32 * kg)) * 4u);
+        return moved(a.A, a.a_bytes, ((unsigned)(m0 + wm0) * (unsigned)a.K + (unsigned)(kbase + k0 + 32 * kg)) * 4u);
     };
     auto at_b = [&](int k0) __attribute__((always_inline)) {
-        return moved(a.B, a.b_bytes, (unsigned)k0 * (unsigned)a.ldb + (unsigned)n0 * ESZ);
+        return moved(a.B, b_bytes, (unsigned)(kbase + k0) * (unsigned)a.ldb + col_bytes((unsigned)n0));
     };
     auto at_s = [&](int k0) __attribute__((always_inline)) {  // scale of (k, n): scales[k * N / 32 + n / 32]
-        return FMT == TML_FMT_Q8_K ? moved(a.scales, a.s_bytes, (unsigned)k0 * ((unsigned)a.N / 8u) + (unsigned)n0 / 8u)
+        return FMT == TML_FMT_Q8_K ? moved(a.scales, a.s_bytes, (unsigned)(kbase + k0) * ((unsigned)a.N / 8u) + (unsigned)n0 / 8u)
                                    : sbf_rsrc(a.B, 0u);
     };
     uint32_t ra[D][TM][8], rb[D][PB][RW];
@@ -221,8 +258,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         return off;
     };
     auto load_a = [&](__amdgpu_buffer_rsrc_t rs, unsigned off, int i, int h, int d) __attribute__((always_inline)) {
-        const uintx4 v =
-            __builtin_amdgcn_raw_buffer_load_b128(rs, off + (unsigned)(16 * i) * (unsigned)a.K * 4u + 64u * h, 0, 0);
+        const uintx4 v = __builtin_amdgcn_raw_buffer_load_b128(
+            rs, AL ? off + (unsigned)(16 * i + 8 * h) * (unsigned)a.K * 4u
+                   : off + (unsigned)(16 * i) * (unsigned)a.K * 4u + 64u * h, 0, 0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) ra[d][i][4 * h + e] = v[e];
     };
@@ -232,9 +270,27 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         const unsigned off = off0 + row * (unsigned)a.ldb;
         if constexpr (FMT == TML_FMT_F32) rb[d][t][kk] = __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0);
         else if constexpr (FMT == TML_FMT_F16) rb[d][t][kk] = __builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0);
-        else {
-            rb[d][t][kk] = __builtin_amdgcn_raw_buffer_load_b8(rs, off, 0, 0);
+        else rb[d][t][kk] = __builtin_amdgcn_raw_buffer_load_b8(rs, off, 0, 0);
+        if constexpr (FMT == TML_FMT_Q8_K) {
             rb[d][t][8 + kk] = __builtin_amdgcn_raw_buffer_load_b32(rsc, s_off[t] + row * ((unsigned)a.N / 8u), 0, 0);
+        }
+    };
+
+    // AL: rows 16 i + 8 h .. + 7 through the wave's own LDS rows (no barrier: one
+    // wave's LDS accesses run in order), 16-byte chunk q of row r in slot q ^ (r % 8).
+    uintx4 *const aw = lds + kARows + wave * (WM * 8);
+    const int slot_aw = lane / 8 * 8 + (lane % 8 ^ lane / 8), slot_ar = c * 8 + (g ^ (c & 7));
+    uint32_t rr[TM][8];
+    auto write_a = [&](int i, int h, int d) __attribute__((always_inline)) {
+        aw[slot_aw + (16 * i + 8 * h) * 8] = (uintx4){ra[d][i][4 * h], ra[d][i][4 * h + 1], ra[d][i][4 * h + 2],
+                                                      ra[d][i][4 * h + 3]};
+    };
+    auto read_a = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uintx4 v = aw[(slot_ar ^ (4 * h)) + 16 * i * 8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) rr[i][4 * h + e] = v[e];
         }
     };
 
@@ -243,7 +299,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     uintx4 av[2][NA][TM], bp[PB][NB];
     auto split_a = [&](int i, int e, int d, int nxt) __attribute__((always_inline)) {
         uint32_t t[NA];
-        sbf_split<NA>(__uint_as_float(ra[d][i][2 * e]), __uint_as_float(ra[d][i][2 * e + 1]), t);
+        sbf_split<NA>(__uint_as_float(AL ? rr[i][2 * e] : ra[d][i][2 * e]),
+                      __uint_as_float(AL ? rr[i][2 * e + 1] : ra[d][i][2 * e + 1]), t);
 #pragma unroll
         for (int p = 0; p < NA; ++p) av[nxt][p][i][e] = t[p];
     };
@@ -255,6 +312,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
             const uint32_t w = rb[d][t][2 * e + z];
             if constexpr (FMT == TML_FMT_F32) x[z] = __uint_as_float(w);
             else if constexpr (FMT == TML_FMT_F16) x[z] = tml_half_bits(w);
+            else if constexpr (FMT == TML_FMT_Q8_0) x[z] = (float)(int8_t)w;
+            else if constexpr (FMT == TML_FMT_Q4_0) x[z] = sbf_int4(w, tid + t * NT);
             else x[z] = (float)(int8_t)w * __uint_as_float(rb[d][t][8 + 2 * e + z]);
         }
         uint32_t v[NB];
@@ -267,12 +326,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     };
 
     // acc holds the hh products, cor the five (four) smaller ones: a slice
-    // rounds the large sum once, and the small terms keep their own.
-    floatx4 acc[TM][TN], cor[TM][TN];
+    // rounds the large sum once, and the small terms keep their own.  (Two terms
+    // of A against int8 or int4 weights share one: the split itself, 2^-17 of a
+    // product, is their error.)
+    floatx4 acc[TM][TN], cor[COR ? TM : 1][COR ? TN : 1];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = cor[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < TN; ++j) {
+            acc[i][j] = (floatx4){0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (COR) cor[i][j] = acc[i][j];
+        }
 
     // One slice: A's operands av[cur] and the LDS stage at sr are multiplied,
     // while B's register set db becomes the stage at sw (two slices on) and A's
@@ -282,13 +346,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // staging follows each group.  A B plane's registers take the next columns --
     // after the last, the first of the next slice at sn -- as soon as the last
     // product that needs it has run.
-    constexpr int NP = NB == 3 ? 6 : 5, JB = TM >= 4 ? 1 : TM >= 2 || TN < 4 ? 2 : 4, kGroups = TN / JB * NP;
+    constexpr int JB = TM >= 4 ? 1 : TM >= 2 || TN < 4 ? 2 : 4, kGroups = TN / JB * NP;
     static_assert(TN % JB == 0, "whole groups of columns");
-    uintx4 bv[NB][JB];
+    // (one plane only: the next columns' registers apart, read a whole group of
+    // columns ahead; group n of the unrolled slices uses bv[n % 2])
+    constexpr int BUF = NB == 1 ? 2 : 1;
+    uintx4 bv[BUF][NB][JB];
     const int slot_r = sbf_slot<SL>(wn0 + c, 4 * kg + g);
-    auto read_b = [&](int p, int j0, int stage) __attribute__((always_inline)) {
+    auto read_b = [&](int buf, int p, int j0, int stage) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < JB; ++j) bv[p][j] = lds[stage + slot_r + p * BN * SL + 16 * SL * (j0 + j)];
+        for (int j = 0; j < JB; ++j) bv[buf][p][j] = lds[stage + slot_r + p * BN * SL + 16 * SL * (j0 + j)];
     };
     // When the staging runs: splitting step v (B's tasks, then A's tiles, four
     // pairs each) after group v kGroups / kSplits; a task's or tile's reloads from
@@ -300,6 +367,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     auto load_at = [](int task, int i) constexpr {
         const int g0 = (4 * task + 3) * kGroups / kSplits + i;
         return g0 < kGroups ? g0 : kGroups - 1;
+    };
+    // (AL: A's rows are read back one group before their first split and written
+    // one before that; their registers are reloaded at once)
+    auto read_a_at = [](int i) constexpr {
+        const int g0 = 4 * (PB + i) * kGroups / kSplits - 1;
+        return g0 > 0 ? g0 : 0;
+    };
+    auto write_a_at = [](int i) constexpr {
+        const int g0 = 4 * (PB + i) * kGroups / kSplits - 2;
+        return g0 > 0 ? g0 : 0;
     };
     auto write_at = [](int t, int p) constexpr {
         const int g0 = (4 * t + 3) * kGroups / kSplits;
@@ -315,22 +392,37 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 #pragma unroll
         for (int j0 = 0; j0 < TN; j0 += JB) {
             constexpr int QA[6] = {0, 1, 2, 0, 1, 0}, QB[6] = {0, 0, 0, 1, 1, 2};
+            const int buf = BUF == 2 ? (TN / JB * cur + j0 / JB) & 1 : 0;
 #pragma unroll
             for (int t = 0; t < NP; ++t) {
 #pragma unroll
                 for (int j = 0; j < JB; ++j)
 #pragma unroll
                     for (int i = 0; i < TM; ++i) {
-                        floatx4 &to = t == 0 ? acc[i][j0 + j] : cor[i][j0 + j];
+                        floatx4 &to = t == 0 || !COR ? acc[i][j0 + j] : cor[COR ? i : 0][COR ? j0 + j : 0];
                         to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, av[cur][QA[t]][i]),
-                                                                     __builtin_bit_cast(bf16x8, bv[QB[t]][j]), to, 0,
+                                                                     __builtin_bit_cast(bf16x8, bv[buf][QB[t]][j]), to, 0,
                                                                      0, 0);
                     }
-                if (t + 1 == NP || QB[t + 1] != QB[t]) {
-                    if (j0 + JB < TN) read_b(QB[t], j0 + JB, sr);
-                    else read_b(QB[t], 0, sn);
+                if (BUF == 2 ? t == 0 : t + 1 == NP || QB[t + 1] != QB[t]) {
+                    if (j0 + JB < TN) read_b(BUF == 2 ? buf ^ 1 : 0, QB[t], j0 + JB, sr);
+                    else read_b(BUF == 2 ? buf ^ 1 : 0, QB[t], 0, sn);
                 }
                 const int gi = j0 / JB * NP + t;
+                if constexpr (AL) {
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+                        if (write_a_at(i) == gi) {
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) {
+                                write_a(i, h, da);
+                                load_a(rsa, a_fresh, i, h, da);
+                            }
+                        }
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+                        if (read_a_at(i) == gi) read_a(i);
+                }
 #pragma unroll
                 for (int v = 0; v < kSplits; ++v)
                     if (split_at(v) == gi) {
@@ -350,7 +442,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int h = 0; h < 2; ++h)
-                        if (load_at(PB + i, h) == gi) load_a(rsa, a_fresh, i, h, da);
+                        if (!AL && load_at(PB + i, h) == gi) load_a(rsa, a_fresh, i, h, da);
 #pragma unroll
                 for (int i = 0; i < TM * JB; ++i) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -367,7 +459,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // is rounded up to whole rounds of U = lcm(2, D) steps (steps past K multiply
     // zeros), so a step's register sets are fixed in the code.
     constexpr int U = D % 2 == 0 ? D : 2 * D;
-    const int nk = ((a.K + BK - 1) / BK + U - 1) / U * U;
+    const int nk = ((kend - kbase + BK - 1) / BK + U - 1) / U * U;
     auto barrier = [&]() __attribute__((always_inline)) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_barrier();
@@ -400,6 +492,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     }
     stage_b(0, 0);
     load_set(false, 0, D * BK);
+    if constexpr (AL) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            write_a(i, 0, 0);
+            write_a(i, 1, 0);
+            read_a(i);
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 4 * TM; ++i) split_a(i / 4, i % 4, 0, 0);
     load_set(true, 0, D * BK);
@@ -407,7 +507,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     load_set(false, 1 % D, (1 + D) * BK);
     barrier();
 #pragma unroll
-    for (int p = 0; p < NB; ++p) read_b(p, 0, 0);
+    for (int p = 0; p < NB; ++p) read_b(0, p, 0, 0);
     int s0 = 0, s1 = kStage, s2 = 2 * kStage;  // the stages of slices kt, kt + 1, kt + 2
     for (int kt0 = 0; kt0 < nk; kt0 += U) {
 #pragma unroll
@@ -424,7 +524,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] += cor[i][j];
+        for (int j = 0; j < TN; ++j)
+            if constexpr (COR) acc[i][j] += cor[i][j];
 
     // ---- epilogue.  The tile's sums go through LDS (free: the loop's last
     // barrier follows every wave's last read) and are written as whole 16-byte
@@ -463,7 +564,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         for (int e = tid; e < BM * BN; e += NT) {
             const int tr = e / BN, row = m0 + tr, col = n0 + e % BN;
             float *const v = &ct[tr * CS + e % BN];
-            if (row < a.M && col < a.N && sbf_suspect(*v)) *v = sbf_fp32_sum<FMT>(a, row, col);
+            if (row < a.M && col < a.N && sbf_suspect(*v)) *v = sbf_fp32_sum<FMT>(a, row, col, kbase, kend);
         }
         __syncthreads();
     }
@@ -471,11 +572,26 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     const int pc = 4 * (tid % CH), tr0 = tid / CH, col = n0 + pc;  // a thread's pieces lie in one column of pieces
     if (tr0 >= RPP || col >= a.N) return;
     const int tr_end = min(BM, a.M - m0);
+    if (a.nsplit > 1) {
+        // raw partial of this split; launch_splitk_reduce adds the splits in
+        // order and runs the epilogue
+        float *const part = a.ws + ((size_t)split * a.M + m0) * a.N + col;
+#pragma unroll 1
+        for (int tr = tr0; tr < tr_end; tr += RPP) {
+            const floatx4 v = *(const floatx4 *)&ct[tr * CS + pc];
+            float *const to = part + (size_t)tr * a.N;
+            if (a.N % 4 == 0) *(floatx4 *)to = v;
+            else
+                for (int q = 0; q < 4 && col + q < a.N; ++q) to[q] = v[q];
+        }
+        return;
+    }
+    auto factor = [&](int n) __attribute__((always_inline)) { return a.colscale ? a.alpha * a.colscale[n] : a.alpha; };
     auto scalar_piece = [&](int tr) {
         const size_t o = (size_t)(m0 + tr) * a.N + col;
 #pragma unroll 1
         for (int q = 0; q < 4 && col + q < a.N; ++q) {
-            float v = a.alpha * ct[tr * CS + pc + q];
+            float v = factor(col + q) * ct[tr * CS + pc + q];
             if (a.beta != 0.0f) v += a.beta * a.C[o + q];
             if (a.bias) v += a.bias[col + q];
             if (a.res) v += a.res[o + q];
@@ -487,6 +603,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         constexpr int ACT = decltype(act_tag)::value, UN = decltype(un_tag)::value;
         floatx4 bias4 = {0.f, 0.f, 0.f, 0.f};
         if (a.bias) bias4 = *(const floatx4 *)(a.bias + col);
+        const floatx4 alpha4 = {factor(col), factor(col + 1), factor(col + 2), factor(col + 3)};
 #pragma unroll 1
         for (int tr = tr0; tr < tr_end; tr += UN * RPP) {
             floatx4 v4[UN], cv[UN], rv[UN];
@@ -510,7 +627,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
                 floatx4 out;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    float v = a.alpha * v4[p][q];
+                    float v = alpha4[q] * v4[p][q];
                     if (a.beta != 0.0f) v += a.beta * cv[p][q];
                     if (a.bias) v += bias4[q];
                     if (a.res) v += rv[p][q];
@@ -550,24 +667,35 @@ constexpr SbfCfg kSbfCfgs[] = {
     {64, 64, 32, 5.1, 0.49, 0.03, 0.83, 1.22},   // four waves of 16 x 64, three workgroups a CU
 };
 constexpr int kSbfNumCfgs = (int)(sizeof(kSbfCfgs) / sizeof(kSbfCfgs[0]));
+// int8 / int4 run the first two only, with these terms
+constexpr SbfCfg kSbfIntCfgs[] = {{256, 128, 32, 6.2, 0.93, 0.32, 0.0, 0.0}, {256, 96, 32, 5.1, 0.83, 0.30, 0.0, 0.0}};
+constexpr int kSbfNumIntCfgs = (int)(sizeof(kSbfIntCfgs) / sizeof(kSbfIntCfgs[0]));
+bool sbf_int(int fmt) { return fmt == TML_FMT_Q8_0 || fmt == TML_FMT_Q4_0; }
+int sbf_num_cfgs(int fmt) { return sbf_int(fmt) ? kSbfNumIntCfgs : kSbfNumCfgs; }
 
 template <int FMT>
 void launch_sbf_cfg(int cfg, unsigned grid, const SbfArgs &a, hipStream_t s) {
-    switch (cfg) {
-        case 0: gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
-        case 1: gemm_sbf_kernel<FMT, 256, 96, 32, 96, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
-        case 2: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 64, 2, 8, 2><<<grid, 512, 0, s>>>(a); break;
-        case 3: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
-        default: gemm_sbf_kernel<FMT, 64, 64, 16, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
+    if constexpr (kSbfInt<FMT>) {
+        // two slices of loads ahead; four measured the same
+        if (cfg == 0) gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 2><<<grid, 512, 0, s>>>(a);
+        else gemm_sbf_kernel<FMT, 256, 96, 32, 96, 32, 1, 8, 2><<<grid, 512, 0, s>>>(a);
+    } else {
+        switch (cfg) {  // (the large tiles' registers hold one slice of loads ahead)
+            case 0: gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
+            case 1: gemm_sbf_kernel<FMT, 256, 96, 32, 96, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
+            case 2: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 64, 2, 8, 2><<<grid, 512, 0, s>>>(a); break;
+            case 3: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
+            default: gemm_sbf_kernel<FMT, 64, 64, 16, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
+        }
     }
 }
 
 }  // namespace
 
 bool gemm_sbf_supported(const MatmulArgs &m) {
-    if (m.fmt != TML_FMT_F32 && m.fmt != TML_FMT_F16 && m.fmt != TML_FMT_Q8_K) return false;
+    if (m.fmt == TML_FMT_Q4_0 && m.N % 2 != 0) return false;
     if (m.M <= kGemvMaxM || m.K <= 0 || m.K % 4 != 0 || ((uintptr_t)m.A % 16) != 0) return false;
-    const uint64_t esz = m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1;
+    const uint64_t esz = m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1;  // (int4: half, bounded as a byte)
     if ((uintptr_t)m.B % esz != 0) return false;
     if (m.fmt == TML_FMT_Q8_K && (m.block != 32 || m.N % 32 != 0 || ((uintptr_t)m.scales % 4) != 0)) return false;
     if (env_int("TML_GEMM_SBF", 1) == 0) return false;
@@ -578,81 +706,126 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 }
 
 // The tile of least modelled time, if that is below `other_us`, the modelled
-// time of the fp32-MFMA kernels' plan (0.97 of it for f32, whose model is the
-// older one).  The terms were fitted to a sweep of the five tiles on MI355X over
+// time of the other kernels' plan (0.95 of it for Q8_K; 1.1 for f32, int8 and int4,
+// whose models run 5-20 % low at these sizes: f32 512x1024x4096 32.4 modelled, 42.8
+// measured, Q8_0 1500x1280x5120 57.6 / 69-73).  The
+// terms were fitted to a sweep of the five tiles on MI355X over
 // M = 200-2048 and N, K = 384-5120 in the three formats (22 shapes; every launch
 // reading one of 8 weight copies).  Measured, us, fp32 MFMA / this kernel's pick:
 //   f32  1500x3840x1280 137 / 80 (256x96), 1500x5120x1280 165 / 95 (256x128),
 //        1500x1280x5120 162 / 115 and 1500x1280x1280 51 / 33 (128x64x64),
 //        512x4096x1024 40.0 / 29.5, 1024x3072x768 47.1 / 35.3 (64x64),
 //        2048x768x3072 83 / 69; where it loses and stays unpicked: 512x1024x1024
-//        13.7 / 21, 512x384x384 5.1 / 10.5, 512x1024x4096 42.8 / 69 (few tiles),
-//        256x3072x1024 18.5 / 21;
+//        13.7 / 21, 512x384x384 5.1 / 10.5, 256x3072x1024 18.5 / 21 (few tiles);
 //   F16  1500x3840x1280 140 / 69, 1500x1280x5120 169 / 105, 512x4096x1024 40.1 /
 //        27.1, 1500x1536x384 19.7 / 17.8, 391x1536x384 11.2 / 9.8;
 //   Q8_K 1500x3840x1280 159 / 82, 1500x1280x5120 185 / 127, 512x4096x1024 44.7 /
 //        31.9, 1024x3072x768 50.2 / 39.7.
 // 2-norm error against 64 bits, the same shapes: 3.7e-7 - 9.9e-7 / 0.9e-7 - 4.5e-7.
-bool pick_sbf(const MatmulArgs &m, double other_us, GemmPlan *p) {
+// int8 / int4 (other_us: the plan of gemm_qbf.hip), us: Q8_0 1500x3840x1280 54-58 /
+// 45.3 (256x96), 1500x5120x1280 57-60 / 50.3, 1500x1280x5120 69-73 / 59.6 (256x128, K
+// split 4); back to back in one encoder layer 42.5 / 38.8, 49.2 / 49.0 and 61.5 /
+// 58.1; where it stays unpicked: 1024x4096x1024 28.0 / 32.7, 1500x1280x1280 25.1 / 38.
+//
+// K is split s ways where the tiles leave CUs idle, at least eight slices a split;
+// the reduce launch costs 2.5 us and the partials' traffic, s M N 8 bytes at 6
+// TB/s (fp32 512x1024x4096, 128x64x64: 77.9 / 47.7 / 39.3 / 33.4 us at s = 1 - 4,
+// the unsplit fp32-MFMA plan 42.8).  A split needs workspace that the other
+// kernel's plan may not: int8 / int4 split at most as often as that plan does
+// (other_split), f32, F16 and Q8_K within the allocation-free entry point's
+// scratch, and not where the caller cannot grow the workspace (m.sbf_split), so a
+// call keeps being served under stream capture and without allocation.
+bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p) {
     constexpr double kCus = 256.0;
-    double best = other_us * (m.fmt == TML_FMT_F32 ? 0.97 : 1.0);
-    int cfg = -1;
-    for (int c = 0; c < kSbfNumCfgs; ++c) {
-        const SbfCfg &t = kSbfCfgs[c];
-        const double rel = m.fmt == TML_FMT_F32 ? 1.0 : m.fmt == TML_FMT_F16 ? t.f16 : t.q8k;
+    const bool is_int = sbf_int(m.fmt);
+    const double mn = (double)m.M * (double)m.N;
+    double best = other_us * (m.fmt == TML_FMT_F32 || is_int ? 1.1 : m.fmt == TML_FMT_Q8_K ? 0.95 : 1.0);
+    int cfg = -1, nsplit = 1;
+    for (int c = 0; c < sbf_num_cfgs(m.fmt); ++c) {
+        const SbfCfg &t = is_int ? kSbfIntCfgs[c] : kSbfCfgs[c];
+        const double rel = m.fmt == TML_FMT_F16 ? t.f16 : m.fmt == TML_FMT_Q8_K ? t.q8k : 1.0;
         if (rel == 0.0) continue;
-        const double w = (double)(((m.M + t.bm - 1) / t.bm) * ((m.N + t.bn - 1) / t.bn)) / kCus;  // tiles a CU
-        const double busy = std::max(0.0, std::min(w, 1.0) - 0.4) * t.busy;
-        double us = t.fixed, slice = t.one + busy;  // one tile a CU
-        if (w > 1.0 && c < 3) {         // one workgroup a CU: whole rounds, each with its own fill and end
-            us += 4.0 * (std::ceil(w) - 1.0);
-            slice *= std::ceil(w);
-        } else if (w > 1.0 && c == 3) {  // two share a CU
-            slice = w <= 2.0 ? 1.25 + 0.2 * (w - 1.0) : 0.75 * w + 0.03;
-        } else if (w > 1.0) {            // three share a CU
-            slice = w <= 2.0 ? 0.69 + 0.16 * (w - 1.0) : w <= 3.0 ? 1.17 + 0.09 * (w - 2.0) : 0.44 * w + 0.02;
-        }
-        us += slice * rel * (double)((m.K + t.bk - 1) / t.bk);
-        if (us < best) {
-            best = us;
-            cfg = c;
+        const int64_t tiles = ((m.M + t.bm - 1) / t.bm) * ((m.N + t.bn - 1) / t.bn);
+        const int64_t slices = (m.K + t.bk - 1) / t.bk;
+        for (int s = 1; s <= 4; ++s) {
+            if (s > 1 && (tiles * s > 256 || slices / s < 8 || !m.sbf_split)) break;
+            if (s > 1 && (is_int ? s > other_split : (double)s * mn > (double)kNoallocPartialFloats)) break;
+            const double w = (double)(tiles * s) / kCus;  // tiles a CU
+            const double busy = std::max(0.0, std::min(w, 1.0) - 0.4) * t.busy;
+            double us = t.fixed, slice = t.one + busy;  // one tile a CU
+            if (w > 1.0 && c < 3) {         // one workgroup a CU: whole rounds, each with its own fill and end
+                us += 4.0 * (std::ceil(w) - 1.0);
+                slice *= std::ceil(w);
+            } else if (w > 1.0) {
+                // two (config 3) or three (4) share a CU: whole rounds of that many, then the rest
+                const double share = c == 3 ? 2.0 : 3.0, rest = w - share * std::floor(w / share);
+                const double whole = std::floor(w / share) * (c == 3 ? 1.50 : 1.32);
+                const double last = rest == 0.0 ? 0.0 : rest <= 1.0 ? t.one : c == 3 ? 1.25 + 0.2 * (rest - 1.0)
+                                    : rest <= 2.0 ? 0.72 + 0.14 * (rest - 1.0) : 1.17 + 0.09 * (rest - 2.0);
+                slice = whole + last;
+            }
+            us += slice * rel * (double)((slices + s - 1) / s);
+            if (s > 1) us += 2.5 + (double)s * mn * 8.0 / 6.0e6;
+            if (us < best) {
+                best = us;
+                cfg = c;
+                nsplit = s;
+            }
         }
     }
     const int forced = env_int("TML_GEMM_SBF_TILE", 0) - 1;
-    if (forced >= 0 && forced < kSbfNumCfgs) cfg = forced;
+    if (forced >= 0 && forced < sbf_num_cfgs(m.fmt)) {
+        cfg = forced;
+        nsplit = std::max(1, env_int("TML_GEMM_SBF_SPLIT", 1));
+    }
     if (cfg < 0) return false;
+    const int64_t bk = kSbfCfgs[cfg].bk, slices = (m.K + bk - 1) / bk;
+    p->spl = (int)((slices + nsplit - 1) / nsplit * bk);
     p->cfg = cfg;
-    p->nsplit = 1;
+    p->nsplit = (int)((m.K + p->spl - 1) / p->spl);
     p->tiles = (int)(((m.M + kSbfCfgs[cfg].bm - 1) / kSbfCfgs[cfg].bm) * ((m.N + kSbfCfgs[cfg].bn - 1) / kSbfCfgs[cfg].bn));
     return true;
 }
 
-Status launch_gemm_sbf(const MatmulArgs &m, const GemmPlan &p, hipStream_t s) {
-    if (!gemm_sbf_supported(m) || p.cfg < 0 || p.cfg >= kSbfNumCfgs)
+Status launch_gemm_sbf(const MatmulArgs &m, const GemmPlan &p, const Workspace &ws, hipStream_t s) {
+    if (!gemm_sbf_supported(m) || p.cfg < 0 || p.cfg >= sbf_num_cfgs(m.fmt))
         return Status::Err(TML_ERR_INVALID_ARG, "split-bf16 GEMM: operands or tile config not supported");
     SbfArgs a;
     a.M = (int)m.M; a.N = (int)m.N; a.K = (int)m.K;
     a.A = m.A; a.B = (const uint8_t *)m.B; a.scales = m.scales;
-    a.ldb = (int)(m.N * (m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1));
+    a.ldb = (int)(m.fmt == TML_FMT_Q4_0 ? m.N / 2 : m.N * (m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1));
+    a.colscale = m.colscale;
     a.bias = m.bias; a.res = m.res; a.C = m.C;
     a.alpha = m.alpha_eff; a.beta = m.beta;
     a.act = m.act;
     a.tail0 = tml_act_tail0((long long)m.M * m.N);
     a.a_bytes = (unsigned)((uint64_t)m.M * (uint64_t)m.K * 4u);
-    a.b_bytes = (unsigned)((uint64_t)m.K * (uint64_t)a.ldb);
     a.s_bytes = m.fmt == TML_FMT_Q8_K ? (unsigned)((uint64_t)m.K * (uint64_t)m.N / 32u * 4u) : 0u;
     a.tiles_m = (int)((m.M + kSbfCfgs[p.cfg].bm - 1) / kSbfCfgs[p.cfg].bm);
     a.tiles_n = (int)((m.N + kSbfCfgs[p.cfg].bn - 1) / kSbfCfgs[p.cfg].bn);
     a.vec_epi = m.N % 4 == 0 && ((uintptr_t)m.C % 16) == 0 && (m.bias == nullptr || ((uintptr_t)m.bias % 16) == 0) &&
-                (m.res == nullptr || ((uintptr_t)m.res % 16) == 0);
-    const int64_t grid = (int64_t)a.tiles_m * a.tiles_n;
+                (m.res == nullptr || ((uintptr_t)m.res % 16) == 0) &&
+                (m.colscale == nullptr || ((uintptr_t)m.colscale % 16) == 0);
+    if (p.nsplit < 1 || p.spl < 1 || p.spl % kSbfCfgs[p.cfg].bk != 0 || (int64_t)p.spl * p.nsplit < m.K ||
+        (int64_t)p.spl * (p.nsplit - 1) >= m.K)
+        return Status::Err(TML_ERR_INVALID_ARG, "split-bf16 GEMM: split plan does not cover K");
+    if (p.nsplit > 1 && (ws.partials == nullptr || ws.partial_floats < (size_t)p.nsplit * (size_t)m.M * (size_t)m.N))
+        return Status::Err(TML_ERR_INVALID_ARG, "split-bf16 GEMM: split-K workspace too small");
+    a.nsplit = p.nsplit;
+    a.spl = p.spl;
+    a.ws = p.nsplit > 1 ? ws.partials : nullptr;
+    const int64_t grid = (int64_t)a.tiles_m * a.tiles_n * p.nsplit;
     if (grid >= ((int64_t)1 << 31)) return Status::Err(TML_ERR_INVALID_SHAPE, "split-bf16 GEMM: grid too large");
     switch (m.fmt) {
         case TML_FMT_F32: launch_sbf_cfg<TML_FMT_F32>(p.cfg, (unsigned)grid, a, s); break;
         case TML_FMT_F16: launch_sbf_cfg<TML_FMT_F16>(p.cfg, (unsigned)grid, a, s); break;
-        default: launch_sbf_cfg<TML_FMT_Q8_K>(p.cfg, (unsigned)grid, a, s); break;
+        case TML_FMT_Q8_K: launch_sbf_cfg<TML_FMT_Q8_K>(p.cfg, (unsigned)grid, a, s); break;
+        case TML_FMT_Q8_0: launch_sbf_cfg<TML_FMT_Q8_0>(p.cfg, (unsigned)grid, a, s); break;
+        case TML_FMT_Q4_0: launch_sbf_cfg<TML_FMT_Q4_0>(p.cfg, (unsigned)grid, a, s); break;
+        default: return Status::Err(TML_ERR_INVALID_FORMAT, "unknown weight format");
     }
     TML_HIP_TRY(hipGetLastError());
+    if (p.nsplit > 1) TML_TRY(launch_splitk_reduce(ws.partials, p.nsplit, m, s));
     return Status::Ok();
 }
 

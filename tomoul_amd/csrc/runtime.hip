@@ -218,8 +218,9 @@ void workspace_need(const MatmulArgs &m, size_t *partial_floats, size_t *counter
 // zeroed, and the zeroing waited for, before this call returns (kernels
 // leave them zero when they finish), so a later call on any stream finds
 // them zero.  Growing allocates, so it is refused while `s` is being
-// captured into a graph: run every captured call once eagerly first.
-Status ensure_workspace(DeviceCtx *c, const MatmulArgs &m, hipStream_t s, Workspace *ws) {
+// captured into a graph: run every captured call once eagerly first.  (A plan of
+// the split-bf16 kernel whose K split alone asks for it runs unsplit instead.)
+Status ensure_workspace(DeviceCtx *c, MatmulArgs &m, hipStream_t s, Workspace *ws) {
     size_t pf = 0, nc = 0;
     workspace_need(m, &pf, &nc);
     if (pf > 0) {
@@ -228,6 +229,10 @@ Status ensure_workspace(DeviceCtx *c, const MatmulArgs &m, hipStream_t s, Worksp
         if (grow_ws || grow_ctr) {
             hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
             TML_HIP_TRY(hipStreamIsCapturing(s, &cap));
+            if (cap != hipStreamCaptureStatusNone && m.sbf_split) {
+                m.sbf_split = false;
+                return ensure_workspace(c, m, s, ws);
+            }
             if (cap != hipStreamCaptureStatusNone)
                 return Status::Err(TML_ERR_INVALID_ARG,
                                    "the split-K workspace must grow during stream capture: run this call once "
@@ -329,8 +334,6 @@ Status gemm_dev(DeviceCtx *c, int fmt, int64_t M, int64_t N, int64_t K, const fl
 // Host code uses the address hipGetSymbolAddress returns for the current
 // device, never the array's name.
 constexpr size_t kScratchBytes = TML_NOALLOC_SCRATCH_BYTES;
-constexpr size_t kScratchCounters = 16384;
-constexpr size_t kScratchPartialOff = 256 + kScratchCounters * sizeof(unsigned);
 static_assert(kScratchPartialOff % 256 == 0 && kScratchPartialOff < kScratchBytes, "scratch layout");
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -389,7 +392,7 @@ Status gemm_dev_noalloc(int fmt, int64_t M, int64_t N, int64_t K, const float *A
     // The plan is the one tml_hip_gemm_ex_dev would run (same kernels, same
     // K splits, same bits); a plan whose partial sums do not fit the static
     // scratch is refused, never replaced by a smaller split.
-    const size_t cap_floats = (kScratchBytes - kScratchPartialOff) / sizeof(float);
+    const size_t cap_floats = kNoallocPartialFloats;
     size_t pf = 0, nc = 0;
     workspace_need(m, &pf, &nc);
     if (pf > cap_floats || nc > kScratchCounters)

@@ -63,6 +63,7 @@ struct MatmulArgs {
     int act = TML_ACT_NONE;  // activation after the bias (TML_ACT_*)
     const float *res = nullptr;  // [M,N] residual added after the bias (may equal C)
     const float *colscale = nullptr;  // [N] per-column factor on A.B (per-channel formats), or nullptr
+    bool sbf_split = true;  // the split-bf16 kernel may split K (needs workspace)
 };
 
 // Activations of the epilogue, restating the reference's CPU code.
@@ -166,6 +167,12 @@ __device__ __forceinline__ void xchg_reset(unsigned *counter) {
     if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Layout of the allocation-free entry point's static scratch: a zero block of 256
+// bytes, the arrival counters, then the split-K partials.
+constexpr size_t kScratchCounters = 16384;
+constexpr size_t kScratchPartialOff = 256 + kScratchCounters * sizeof(unsigned);
+constexpr size_t kNoallocPartialFloats = (TML_NOALLOC_SCRATCH_BYTES - kScratchPartialOff) / sizeof(float);
+
 // Split-K workspace handed to kernels that reduce across workgroups.
 struct Workspace {
     float *partials = nullptr;      // nsplit * M * N floats
@@ -185,7 +192,7 @@ struct GemmPlan {
     int spl = 0;       // BK-slices per split
     int tiles = 0;
     bool fused = false;  // split-K partials combined in the GEMM kernel (no reduce launch)
-    bool sbf = false;    // f32 / F16 / Q8_K on the bf16 matrix cores (gemm_sbf.hip; cfg its tile)
+    bool sbf = false;    // the split-bf16 kernel (gemm_sbf.hip; cfg its tile, spl in k)
     bool qbf = false;    // Q8_0 / Q4_0 on the bf16 matrix cores (gemm_qbf.hip; cfg, nsplit, spl its plan)
 };
 GemmPlan plan_gemm(const MatmulArgs &a);
@@ -204,14 +211,16 @@ Status launch_gemm_f32_dma(const MatmulArgs &a, const GemmPlan &p, const Workspa
 // p->cfg / nsplit / spl; K splits write nsplit * M * N partial floats that
 // launch_splitk_reduce sums.
 bool gemm_qbf_supported(const MatmulArgs &a);
-void pick_qbf(const MatmulArgs &a, GemmPlan *p);
+// Returns the plan's modelled time (0 where a rule, not the model, chose it).
+double pick_qbf(const MatmulArgs &a, GemmPlan *p);
 Status launch_gemm_qbf(const MatmulArgs &a, const GemmPlan &p, const Workspace &ws, hipStream_t s);
-// f32 / F16 / Q8_K GEMM on the bf16 matrix cores (gemm_sbf.hip): M >
-// kGemvMaxM, K % 4 == 0, 16-byte aligned A.  pick_sbf is false where the
-// fp32-MFMA kernels, at a modelled other_us, are the faster choice.
+// GEMM on the bf16 matrix cores with the operands split into bf16 terms
+// (gemm_sbf.hip): M > kGemvMaxM, K % 4 == 0, 16-byte aligned A.  pick_sbf is false
+// where the other kernels, at a modelled other_us with other_split K splits, are
+// the faster choice.
 bool gemm_sbf_supported(const MatmulArgs &a);
-bool pick_sbf(const MatmulArgs &a, double other_us, GemmPlan *p);
-Status launch_gemm_sbf(const MatmulArgs &a, const GemmPlan &p, hipStream_t s);
+bool pick_sbf(const MatmulArgs &a, double other_us, int other_split, GemmPlan *p);
+Status launch_gemm_sbf(const MatmulArgs &a, const GemmPlan &p, const Workspace &ws, hipStream_t s);
 // C = act(alpha * sum of the nsplit [M,N] partials (in split order) * colscale + beta * C + bias + res).
 Status launch_splitk_reduce(const float *partials, int nsplit, const MatmulArgs &a, hipStream_t s);
 void gemm_dma_workspace_need(const MatmulArgs &a, const GemmPlan &p, size_t *partial_floats, size_t *counters);
