@@ -460,19 +460,6 @@ int pick_cfg(int64_t M, int64_t N, int cus) {
     return best;
 }
 
-int device_cus() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            cus = n;
-        else
-            cus = 256;
-    }
-    return cus;
-}
-
 // Direct-copy fp32 kernel: pick (tile, K splits) with the smallest modelled
 // time.  A CU runs its share of the units (tile x split); with one unit per
 // CU a slice costs t_one, with several resident at once their slices overlap
@@ -648,10 +635,7 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
     // the bf16 matrix-core kernel whenever its layout conditions hold
     // (gemm_qbf.hip), unless TML_GEMM_QBF=0 or an override asks for a tile or
     // K split of the fp32-MFMA kernels below (tests of those kernels).
-    auto set = [](const char *k) {
-        const char *v = std::getenv(k);
-        return v != nullptr && *v != '\0';
-    };
+    auto set = [](const char *k) { return env_text(k) != nullptr; };
     const bool fp32_forced = set("TML_GEMM_DMA_Q") || set("TML_GEMM_TILE") || set("TML_GEMM_DMA_TILE") ||
                              set("TML_GEMM_SPLIT");
     if (!fp32_forced && gemm_qbf_supported(m)) {
@@ -730,7 +714,7 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
 }
 
 void gemm_workspace_need(const MatmulArgs &m, size_t *partial_floats, size_t *counters) {
-    const GemmPlan p = plan_gemm(m);
+    const GemmPlan p = m.plan != nullptr ? *m.plan : plan_gemm(m);
     *partial_floats = 0;
     *counters = 0;
     if ((p.qbf || p.sbf) && p.nsplit > 1) *partial_floats = (size_t)p.nsplit * (size_t)m.M * (size_t)m.N;
@@ -758,8 +742,7 @@ bool plan_forced() {
                                        "TML_GEMM_DMA",      "TML_GEMM_FUSED", "TML_GEMM_XCDPART", "TML_GEMM_XCD",
                                        "TML_GEMM_GROUPM",   "TML_GEMM_QBF_TILE", "TML_GEMM_QBF_SPLIT"};
     for (const char *k : keys) {
-        const char *v = std::getenv(k);
-        if (v != nullptr && *v != '\0') return true;
+        if (env_text(k) != nullptr) return true;
     }
     return false;
 }
@@ -774,7 +757,7 @@ Status launch_gemm_mfma(const MatmulArgs &m, const Workspace &ws, hipStream_t s)
         return Status::Err(TML_ERR_INVALID_ARG,
                            "forced GEMM plans (TML_GEMM_* overrides) are refused above M*N*K = 512*1024*4096, "
                            "the largest size the tests run them at");
-    const GemmPlan p = plan_gemm(m);
+    const GemmPlan p = m.plan != nullptr ? *m.plan : plan_gemm(m);
     // TML_REQUIRE_SPLIT=1 (tests): refuse a plan that does not split K
     if (!((p.qbf || p.dma || p.sbf) && p.nsplit > 1) && env_int("TML_REQUIRE_SPLIT", 0) == 1)
         return Status::Err(TML_ERR_INVALID_ARG, "TML_REQUIRE_SPLIT=1: this call's plan does not split K");

@@ -557,11 +557,7 @@ void launch_qbf_cfg(int cfg, unsigned grid, const QbfArgs &a, hipStream_t s) {
 //     53.1 us at 1500x3840x1280, 67.6 at 1500x5120x1280 and 35.0 at
 //     1024x4096x1024, 9-13 us above the model.
 double pick_qbf(const MatmulArgs &m, GemmPlan *p) {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-    }
+    const int cus = device_cus();
     const int64_t nk = (m.K + 31) / 32;
     auto tiles_of = [&](int c) {
         return ((m.M + kQbfCfgs[c].bm - 1) / kQbfCfgs[c].bm) * ((m.N + kQbfCfgs[c].bn - 1) / kQbfCfgs[c].bn);

@@ -455,19 +455,6 @@ int elems_per_lane(int fmt, int lw) {
 
 bool is_aligned(const void *p, size_t n) { return ((uintptr_t)p % n) == 0; }
 
-int gemv_cus() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            cus = n;
-        else
-            cus = 256;
-    }
-    return cus;
-}
-
 // Segment width: the narrowest segment of at least one 128-byte line per
 // row that wastes little of the last segment; narrower segments mean fewer
 // K splits (less partial traffic) at the cost of more shuffle steps.
@@ -529,7 +516,7 @@ GemvPlan make_plan(const MatmulArgs &m) {
     // -> 5.46 / 6.05 / 7.21 us.  Slower at M = 8 (8.3 -> 10.5 us) and for
     // Q4_0 and f32 at their layer shapes.
     if (m.fmt == TML_FMT_Q8_0 && aligned && p.mr <= 4 && m.K <= (int64_t)kWaves * 64 * kU &&
-        m.N / p.e >= gemv_cus())
+        m.N / p.e >= device_cus())
         lpr = 1;
     const int forced_lpr = env_int("TML_GEMV_LPR", 0);
     if (forced_lpr == 4 || forced_lpr == 8 || forced_lpr == 16 || forced_lpr == 32 || forced_lpr == 64)
@@ -544,7 +531,7 @@ GemvPlan make_plan(const MatmulArgs &m) {
     // K splits: enough workgroups for about two per CU, but at most
     // kMaxSplit per segment -- every split adds an arrival on the segment's
     // counter, and those atomics serialise.
-    const int cus = gemv_cus();
+    const int cus = device_cus();
     int64_t nb = 1;
     const int forced_nb = env_int("TML_GEMV_NB", 0);
     if (forced_nb > 0) {

@@ -700,11 +700,7 @@ Status launch_gemv_t(int fmt, int64_t M, int64_t N, int64_t K, const float *A, c
     ka.act = act;
     ka.res = res;
     ka.tail0 = tail0;
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-    }
+    const int cus = device_cus();
     const bool xvec = (K % 4 == 0) && ((uintptr_t)A % 16 == 0);
     // The direct kernel holds a chunk's activations for every row in
     // registers (MR * E <= 64); beyond that, and where TML_GEMVT_LDS=1 asks

@@ -446,11 +446,7 @@ Status launch_gemv_tm(int fmt, int64_t M, int64_t N, int64_t K, const float *A, 
     ka.act = act; ka.res = res; ka.tail0 = tail0;
     ka.wbytes = (unsigned)(N * ldt);
     ka.xbytes = (unsigned)(M * K * 4);
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-    }
+    const int cus = device_cus();
     // Two 16-column tiles a workgroup at M > 4 where one tile each would
     // leave some CU two workgroups: each CU then stages the activations once
     // for 32 columns instead of twice for 16 (1280x5120 Q4_0, M = 8: 5.48

@@ -367,11 +367,7 @@ Status launch_gemv_x(int fmt, int64_t M, int64_t N, int64_t K, const float *A, c
         return Status::Err(TML_ERR_INVALID_ARG, "staged-activation GEMV: prepared layout or alignment");
     if (N * ldt >= ((int64_t)1 << 31))
         return Status::Err(TML_ERR_INVALID_SHAPE, "staged-activation GEMV: weight too large");
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) cus = n;
-    }
+    const int cus = device_cus();
     XPlan p;
     if (!x_plan(fmt, M, N, K, cus, &p)) return Status::Err(TML_ERR_INVALID_ARG, "staged-activation GEMV: no plan");
     GemvXArgs ka;

@@ -7,7 +7,10 @@
 // (or reuse a registered weight), launch, download C, synchronise.
 // tml_hip_gemm_ex_dev_noalloc is the device-pointer entry point for callers
 // that cannot allocate: its split-K scratch is a static device array.
+#include <unistd.h>
+
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -28,10 +31,44 @@ Status hip_status(hipError_t e, const char *what) {
     return Status::Err(code, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-int env_int(const char *name, int dflt) {
+namespace {
+thread_local int t_env = -1;  // inside an EnvCall: whether the environment holds a TML_ name
+}  // namespace
+
+EnvCall::EnvCall() : outer_(t_env) {
+    if (t_env >= 0) return;
+    t_env = 0;
+    for (char **e = environ; e != nullptr && *e != nullptr; ++e)
+        if (std::strncmp(*e, "TML_", 4) == 0) {
+            t_env = 1;
+            break;
+        }
+}
+EnvCall::~EnvCall() { t_env = outer_; }
+
+const char *env_text(const char *name) {
+    if (t_env == 0) return nullptr;
     const char *v = std::getenv(name);
-    if (v == nullptr || *v == '\0') return dflt;
-    return std::atoi(v);
+    return v != nullptr && *v != '\0' ? v : nullptr;
+}
+
+int env_int(const char *name, int dflt) {
+    const char *v = env_text(name);
+    return v != nullptr ? std::atoi(v) : dflt;
+}
+
+int device_cus() {
+    static std::atomic<int> known{0};
+    int cus = known.load(std::memory_order_relaxed);
+    if (cus == 0) {
+        int dev = 0, n = 0;
+        cus = 256;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+            cus = n;
+        known.store(cus, std::memory_order_relaxed);
+    }
+    return cus;
 }
 
 namespace {
@@ -168,10 +205,18 @@ std::unordered_map<int, DeviceCtx *> g_ctx;
 Status scratch_setup(hipStream_t s, void **base);
 
 Status current_ctx(DeviceCtx **out) {
-    int n = 0;
+    // (a device that has a context exists: no need to count them again)
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess) {
+        std::lock_guard<std::mutex> lk(g_mu);
+        auto it = g_ctx.find(dev);
+        if (it != g_ctx.end()) {
+            *out = it->second;
+            return Status::Ok();
+        }
+    }
     hipError_t e = hipGetDeviceCount(&n);
     if (e != hipSuccess || n <= 0) return Status::Err(TML_ERR_NO_DEVICE, "no HIP device available");
-    int dev = 0;
     TML_HIP_TRY(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_ctx.find(dev);
@@ -206,6 +251,13 @@ Status current_ctx(DeviceCtx **out) {
     return Status::Ok();
 }
 
+// The GEMM's plan, made once for the workspace and the launch.
+void keep_plan(MatmulArgs &m, GemmPlan *plan) {
+    if (m.M <= kGemvMaxM) return;
+    *plan = plan_gemm(m);
+    m.plan = plan;
+}
+
 // Split-K workspace (partial sums and arrival counters) this problem needs.
 void workspace_need(const MatmulArgs &m, size_t *partial_floats, size_t *counters) {
     *partial_floats = 0;
@@ -231,6 +283,7 @@ Status ensure_workspace(DeviceCtx *c, MatmulArgs &m, hipStream_t s, Workspace *w
             TML_HIP_TRY(hipStreamIsCapturing(s, &cap));
             if (cap != hipStreamCaptureStatusNone && m.sbf_split) {
                 m.sbf_split = false;
+                if (m.plan != nullptr) *m.plan = plan_gemm(m);
                 return ensure_workspace(c, m, s, ws);
             }
             if (cap != hipStreamCaptureStatusNone)
@@ -319,6 +372,9 @@ Status gemm_dev(DeviceCtx *c, int fmt, int64_t M, int64_t N, int64_t K, const fl
     TML_TRY(matmul_args(fmt, M, N, K, A, B, scale, scales, block, bias, C, alpha, beta, act, res, &m, &empty));
     if (empty) return Status::Ok();
     m.zero = c->zero.p;
+    const EnvCall env;
+    GemmPlan plan;
+    keep_plan(m, &plan);
     Workspace ws;
     TML_TRY(ensure_workspace(c, m, s, &ws));
     return launch_matmul(m, ws, s);
@@ -393,6 +449,9 @@ Status gemm_dev_noalloc(int fmt, int64_t M, int64_t N, int64_t K, const float *A
     // K splits, same bits); a plan whose partial sums do not fit the static
     // scratch is refused, never replaced by a smaller split.
     const size_t cap_floats = kNoallocPartialFloats;
+    const EnvCall env;
+    GemmPlan plan;
+    keep_plan(m, &plan);
     size_t pf = 0, nc = 0;
     workspace_need(m, &pf, &nc);
     if (pf > cap_floats || nc > kScratchCounters)
@@ -457,6 +516,7 @@ Status make_prepared(DeviceCtx *c, int fmt, int64_t K, int64_t N, const void *B,
 Status gemm_prepared(DeviceCtx *c, const Prepared *p, int64_t M, const float *A, const float *bias, float *C,
                      float alpha, float beta, hipStream_t s, int act = TML_ACT_NONE,
                      const float *res = nullptr) {
+    const EnvCall env;
     if (M < 0) return Status::Err(TML_ERR_INVALID_SHAPE, "negative matrix dimension");
     if (!valid_act(act)) return Status::Err(TML_ERR_INVALID_ARG, "unknown activation");
     if (M == 0 || p->N == 0) return Status::Ok();
