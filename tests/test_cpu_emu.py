@@ -348,6 +348,10 @@ def test_sbf_cases(emu):
     for tile in range(1, 6):
         cases += [f"gemm 0 130 97 516 br TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT=3",
                   f"noalloc 3 257 192 260 b TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT=2"]
+        # K of no whole 16-byte load: rows of A start on any dword, the last load crosses A's end
+        cases += [f"gemm {fmt} {M} {N} {K} br TML_GEMM_SBF_TILE={tile}" for fmt in (F32, F16, Q8_K)
+                  for (M, N, K) in [(130, 96, 513), (17, 64, 31), (257, 160, 70)]]
+    cases += ["gemm 0 130 97 515 b", "gemm 4 33 131 1001 b"]
     cases += ["gemm 0 1500 3840 64 b", "gemm 4 1500 3840 64 e", "gemm 3 1500 3840 64 br", "gemm 0 100 1001 388 bt"]
     outs, fails = run_cases(emu, cases)
     assert not fails and not _err_lines(outs), (fails, _err_lines(outs)[:3])

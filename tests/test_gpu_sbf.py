@@ -98,6 +98,31 @@ def test_sbf_default_plan_epilogue(orc, fmt, m, n, k):
         assert np.max(np.abs(c - ref)) <= 1e-6 * max(1.0, np.max(np.abs(ref))), act
 
 
+@pytest.mark.parametrize("fmt", [_abi.FMT_F32, _abi.FMT_F16, _abi.FMT_Q8_K])
+@pytest.mark.parametrize("tile,split", [(t, 1) for t in TILES] + [(3, 2), (5, 3)])
+def test_sbf_any_k(orc, env, tile, split, fmt):
+    # K of no whole 16-byte load: rows of A start on any dword, and the last row's
+    # last load crosses the end of A
+    env["TML_GEMM_SBF_TILE"], env["TML_GEMM_SBF_SPLIT"] = str(tile), str(split)
+    for (m, n, k) in [(9, 32, 1), (33, 160, 35), (257, 288, 518), (130, 96, 1033)]:
+        a, bias = synth.normal_matrix(81 + m, m, k), synth.normal(82, n, 0.0, 0.02)
+        q, scales, w = weight(orc, fmt, synth.normal_matrix(83, k, n, 0.02))
+        check(run(fmt, m, n, k, a, q, scales, bias=bias), a, w, bias.astype(np.float64))
+
+
+def test_sbf_unaligned_a():
+    # A on any dword, K odd or even, the planner's own choice
+    import torch
+    for (m, n, k, off) in [(40, 130, 255, 1), (300, 512, 256, 2), (77, 97, 1030, 3)]:
+        gen = torch.Generator(device="cuda").manual_seed(k)
+        flat = torch.randn(m * k + off, generator=gen, device="cuda")
+        a, w = flat[off:].reshape(m, k), torch.randn(k, n, generator=gen, device="cuda") * 0.02
+        c = torch.zeros(m, n, device="cuda")
+        _abi.gemm_dev(_abi.FMT_F32, m, n, k, a.data_ptr(), w.data_ptr(), c.data_ptr(),
+                      stream=torch.cuda.current_stream().cuda_stream)
+        check(c.cpu().numpy(), a.cpu().numpy(), w.cpu().numpy())
+
+
 @pytest.mark.parametrize("tile", TILES)
 def test_sbf_inf_nan(orc, env, tile):
     env["TML_GEMM_SBF_TILE"] = str(tile)

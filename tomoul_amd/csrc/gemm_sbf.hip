@@ -52,7 +52,7 @@ constexpr int kSbfXcd = 8;  // XCDs of an MI355X: workgroups are dealt to them r
 
 struct SbfArgs {
     int M, N, K;
-    const float *A;         // [M,K], K % 4 == 0, 16-byte aligned
+    const float *A;         // [M,K], 4-byte aligned (int8 / int4: K % 4 == 0, 16-byte aligned)
     const uint8_t *B;       // [K,N]: f32, binary16, int8, or int4 two a byte (even n in the low nibble)
     const float *scales;    // Q8_K block scales (32 elements each, N % 32 == 0)
     int ldb;                // bytes per B row
@@ -694,7 +694,11 @@ void launch_sbf_cfg(int cfg, unsigned grid, const SbfArgs &a, hipStream_t s) {
 
 bool gemm_sbf_supported(const MatmulArgs &m) {
     if (m.fmt == TML_FMT_Q4_0 && m.N % 2 != 0) return false;
-    if (m.M <= kGemvMaxM || m.K <= 0 || m.K % 4 != 0 || ((uintptr_t)m.A % 16) != 0) return false;
+    if (m.M <= kGemvMaxM || m.K <= 0) return false;
+    // A's 16-byte loads need 4-byte alignment only, and a load that crosses the end
+    // of A is checked dword by dword: any K serves.  (Int8 / int4: the layouts that
+    // the kernel they compete with takes.)
+    if (sbf_int(m.fmt) ? m.K % 4 != 0 || ((uintptr_t)m.A % 16) != 0 : ((uintptr_t)m.A % 4) != 0) return false;
     const uint64_t esz = m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1;  // (int4: half, bounded as a byte)
     if ((uintptr_t)m.B % esz != 0) return false;
     if (m.fmt == TML_FMT_Q8_K && (m.block != 32 || m.N % 32 != 0 || ((uintptr_t)m.scales % 4) != 0)) return false;
@@ -726,6 +730,13 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 // 45.3 (256x96), 1500x5120x1280 57-60 / 50.3, 1500x1280x5120 69-73 / 59.6 (256x128, K
 // split 4); back to back in one encoder layer 42.5 / 38.8, 49.2 / 49.0 and 61.5 /
 // 58.1; where it stays unpicked: 1024x4096x1024 28.0 / 32.7, 1500x1280x1280 25.1 / 38.
+//
+// Layouts no other kernel has wide loads for (K % 4 != 0, odd N, A on a 4-byte
+// boundary) always come here: the register-staged kernel reads them element by
+// element and does not split K.  Measured, us, that kernel / this one: f32
+// 9x4001x401 19.1 / 12.2, 60x401x399 20.6 / 15.3, 278x1340x2235 92 / 22.9,
+// 1500x1537x383 45.9 / 30.3, 2500x3001x1999 501 / 186, 30x777x4999 188 / 30.3; F16
+// 700x1111x1777 134 / 32.9, 20x3333x501 32.3 / 11.7.
 //
 // K is split s ways where the tiles leave CUs idle, at least eight slices a split;
 // the reduce launch costs 2.5 us and the partials' traffic, s M N 8 bytes at 6
