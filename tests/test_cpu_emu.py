@@ -351,6 +351,10 @@ def test_sbf_cases(emu):
         # K of no whole 16-byte load: rows of A start on any dword, the last load crosses A's end
         cases += [f"gemm {fmt} {M} {N} {K} br TML_GEMM_SBF_TILE={tile}" for fmt in (F32, F16, Q8_K)
                   for (M, N, K) in [(130, 96, 513), (17, 64, 31), (257, 160, 70)]]
+    for tile in (2, 3, 5):
+        cases += [f"gemm {fmt} {M} {N} {K} br TML_GEMM_SBF_TILE={tile}" for fmt in (Q8_0, Q4_0, Q8_0_PC)
+                  for (M, N, K) in [(130, 98, 513), (17, 64, 33), (257, 162, 71)]]
+        cases += [f"gemm {Q8_0} 70 33 517 br TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT=2"]
     cases += ["gemm 0 130 97 515 b", "gemm 4 33 131 1001 b"]
     cases += ["gemm 0 1500 3840 64 b", "gemm 4 1500 3840 64 e", "gemm 3 1500 3840 64 br", "gemm 0 100 1001 388 bt"]
     outs, fails = run_cases(emu, cases)

@@ -196,6 +196,28 @@ def test_sbf_int(orc, env, tile, split):
             check(c, a, np.asarray(deq, np.float32).reshape(k, n), bias.astype(np.float64), terms=2)
 
 
+@pytest.mark.parametrize("tile,split", [(0, 1), (2, 1), (3, 1), (3, 2), (5, 1), (5, 3)])
+def test_sbf_int_exact(orc, env, tile, split):
+    # int8 / int4 outside gemm_qbf.hip's layouts (odd N, K % 8 != 0): three terms of
+    # A, within the fp32 products' bound; 0: the planner's own choice
+    if tile:
+        env["TML_GEMM_SBF_TILE"], env["TML_GEMM_SBF_SPLIT"] = str(tile), str(split)
+    for (m, n, k) in [(9, 33, 5), (300, 130, 517), (257, 97, 1288), (70, 64, 1026)]:
+        a, bias = synth.normal_matrix(91 + m, m, k), synth.normal(92, n, 0.0, 0.02)
+        w = synth.normal_matrix(93, k, n, 0.02)
+        q, s = orc.quantize_q8(w)
+        qc, sc = orc.quantize_q8_cols(w)
+        check(run(_abi.FMT_Q8_0, m, n, k, a, q, None, scale=s, bias=bias), a, orc.dequantize_q8(q, s).reshape(k, n),
+              bias.astype(np.float64))
+        check(run(_abi.FMT_Q8_0_PC, m, n, k, a, qc, sc, bias=bias), a,
+              np.asarray(orc.dequantize_cols(_abi.FMT_Q8_0_PC, qc, sc, k, n), np.float32).reshape(k, n),
+              bias.astype(np.float64))
+        if n % 2 == 0:
+            p, s4 = orc.quantize_q4(w)
+            check(run(_abi.FMT_Q4_0, m, n, k, a, p, None, scale=s4, bias=bias), a,
+                  orc.dequantize_q4(p, k * n, s4).reshape(k, n), bias.astype(np.float64))
+
+
 @pytest.mark.parametrize("tile", [1, 2])
 def test_sbf_int_inf_nan(orc, env, tile):
     env["TML_GEMM_SBF_TILE"] = str(tile)

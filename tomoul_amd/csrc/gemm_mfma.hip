@@ -704,8 +704,12 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
     // asks for one of the fp32-MFMA kernels.
     const bool other_forced = fp32_forced || set("TML_GEMM_DMA") || set("TML_GEMM_FUSED") || set("TML_GEMM_XCDPART") ||
                               set("TML_GEMM_XCD") || set("TML_GEMM_GROUPM");
+    // Int8 / int4 outside gemm_qbf.hip's layouts likewise, where the register-staged
+    // kernel would read them element by element (its own override, TML_GEMM_QBF, aside).
     GemmPlan q;
-    if (!other_forced && m.fmt != TML_FMT_Q8_0 && m.fmt != TML_FMT_Q4_0 && gemm_sbf_supported(m) &&
+    const bool is_int = m.fmt == TML_FMT_Q8_0 || m.fmt == TML_FMT_Q4_0;
+    const bool int_ok = m.K % 4 != 0 || m.N % 8 != 0 || !aligned(m.A, 16) || !aligned(m.B, m.fmt == TML_FMT_Q4_0 ? 4 : 8);
+    if (!other_forced && (!is_int || (int_ok && !set("TML_GEMM_QBF"))) && gemm_sbf_supported(m) &&
         pick_sbf(m, other_us, p.nsplit, &q)) {
         q.sbf = true;
         return q;

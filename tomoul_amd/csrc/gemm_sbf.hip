@@ -19,7 +19,9 @@
 // against 64 bits is 0.9e-7 - 4.5e-7 over the shapes at pick_sbf, theirs 3.7e-7 -
 // 9.9e-7.
 // Int8 and int4 weights are exact in bf16 and A takes two terms, |x - hi - lo| <=
-// 2^-17 |x|: two products, the arithmetic of gemm_qbf.hip.
+// 2^-17 |x|: two products, the arithmetic of gemm_qbf.hip.  Outside that kernel's
+// layouts, where the fp32 matrix cores' general kernel ran, A takes three terms and
+// the products are three: fp32 precision as before.
 //
 // Bound: the matrix cores, at the clock the power limit leaves them.  At
 // 1500x5120x1280 (240 tiles of 256x128) the main loop keeps them 82 % busy, at
@@ -52,7 +54,7 @@ constexpr int kSbfXcd = 8;  // XCDs of an MI355X: workgroups are dealt to them r
 
 struct SbfArgs {
     int M, N, K;
-    const float *A;         // [M,K], 4-byte aligned (int8 / int4: K % 4 == 0, 16-byte aligned)
+    const float *A;         // [M,K], 4-byte aligned
     const uint8_t *B;       // [K,N]: f32, binary16, int8, or int4 two a byte (even n in the low nibble)
     const float *scales;    // Q8_K block scales (32 elements each, N % 32 == 0)
     int ldb;                // bytes per B row
@@ -103,14 +105,19 @@ __device__ __forceinline__ int sbf_slot(int r, int s) {
 }
 
 // bf16 terms of A and B, and the pairs of them multiplied.
+// Int8 / int4 at the fp32 products' precision (kSbfExact added to the format): three
+// terms of A, three products.
+constexpr int kSbfExact = 64;
+template <int FMT>
+constexpr int kSbfStored = FMT & ~kSbfExact;  // B's format in memory
 template <int FMT>
 constexpr bool kSbfInt = FMT == TML_FMT_Q8_0 || FMT == TML_FMT_Q4_0;
 template <int FMT>
 constexpr int kSbfPlanesA = kSbfInt<FMT> ? 2 : 3;
 template <int FMT>
-constexpr int kSbfPlanesB = kSbfInt<FMT> ? 1 : FMT == TML_FMT_F16 ? 2 : 3;
+constexpr int kSbfPlanesB = kSbfInt<FMT> || FMT >= kSbfExact ? 1 : FMT == TML_FMT_F16 ? 2 : 3;
 template <int FMT>
-constexpr int kSbfProducts = kSbfInt<FMT> ? 2 : FMT == TML_FMT_F16 ? 5 : 6;
+constexpr int kSbfProducts = kSbfInt<FMT> ? 2 : FMT >= kSbfExact ? 3 : FMT == TML_FMT_F16 ? 5 : 6;
 // The int4 value of column n in the byte that holds it.
 __device__ __forceinline__ float sbf_int4(uint32_t byte, int n) {
     return (float)((int32_t)(byte << ((n & 1) ? 24 : 28)) >> 28);
@@ -121,8 +128,8 @@ template <int FMT>
 __device__ __forceinline__ float sbf_b(const SbfArgs &a, int k, int n) {
     if constexpr (FMT == TML_FMT_F32) return ((const float *)a.B)[(size_t)k * a.N + n];
     else if constexpr (FMT == TML_FMT_F16) return tml_half_bits(((const uint16_t *)a.B)[(size_t)k * a.N + n]);
-    else if constexpr (FMT == TML_FMT_Q8_0) return (float)((const int8_t *)a.B)[(size_t)k * a.N + n];
-    else if constexpr (FMT == TML_FMT_Q4_0) return sbf_int4(a.B[(size_t)k * a.ldb + n / 2], n);
+    else if constexpr (kSbfStored<FMT> == TML_FMT_Q8_0) return (float)((const int8_t *)a.B)[(size_t)k * a.N + n];
+    else if constexpr (kSbfStored<FMT> == TML_FMT_Q4_0) return sbf_int4(a.B[(size_t)k * a.ldb + n / 2], n);
     else return (float)((const int8_t *)a.B)[(size_t)k * a.N + n] * a.scales[((size_t)k * a.N + n) >> 5];
 }
 
@@ -218,7 +225,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // outputs.  (A value there that is not finite makes its sum a NaN, which the
     // epilogue recomputes.)
     constexpr unsigned ESZ = FMT == TML_FMT_F32 ? 4u : FMT == TML_FMT_F16 ? 2u : 1u;
-    auto col_bytes = [](unsigned n) constexpr { return FMT == TML_FMT_Q4_0 ? n / 2u : n * ESZ; };
+    auto col_bytes = [](unsigned n) constexpr { return kSbfStored<FMT> == TML_FMT_Q4_0 ? n / 2u : n * ESZ; };
     const unsigned b_bytes = (unsigned)kend * (unsigned)a.ldb;
     // A: AL loads 8 rows of 128 bytes an instruction (lane / 8, lane % 8), else 16
     // rows' 16-byte pieces in the MFMA's layout (c, g)
@@ -312,8 +319,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
             const uint32_t w = rb[d][t][2 * e + z];
             if constexpr (FMT == TML_FMT_F32) x[z] = __uint_as_float(w);
             else if constexpr (FMT == TML_FMT_F16) x[z] = tml_half_bits(w);
-            else if constexpr (FMT == TML_FMT_Q8_0) x[z] = (float)(int8_t)w;
-            else if constexpr (FMT == TML_FMT_Q4_0) x[z] = sbf_int4(w, tid + t * NT);
+            else if constexpr (kSbfStored<FMT> == TML_FMT_Q8_0) x[z] = (float)(int8_t)w;
+            else if constexpr (kSbfStored<FMT> == TML_FMT_Q4_0) x[z] = sbf_int4(w, tid + t * NT);
             else x[z] = (float)(int8_t)w * __uint_as_float(rb[d][t][8 + 2 * e + z]);
         }
         uint32_t v[NB];
@@ -657,21 +664,28 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 struct SbfCfg {
     int bm, bn, bk;
     double fixed, one, busy;
-    double f16, q8k;  // the slice's cost in these formats, relative to f32 (0: not used)
+    double f16, q8k, exact;  // the slice's cost in F16, Q8_K and exact int8 / int4, relative to f32 (0: not used)
 };
 constexpr SbfCfg kSbfCfgs[] = {
-    {256, 128, 32, 9.7, 1.58, 1.25, 0.86, 0.0},  // eight waves of 32 x 128
-    {256, 96, 32, 8.9, 1.33, 0.95, 0.86, 1.05},  // eight waves of 32 x 96
-    {128, 64, 64, 8.2, 1.13, 0.37, 0.91, 1.09},  // two wave groups of four 32 x 64
-    {128, 64, 32, 6.4, 0.67, 0.13, 0.86, 1.12},  // four waves of 32 x 64, two workgroups a CU
-    {64, 64, 32, 5.1, 0.49, 0.03, 0.83, 1.22},   // four waves of 16 x 64, three workgroups a CU
+    {256, 128, 32, 9.7, 1.58, 1.25, 0.86, 0.0, 0.0},  // eight waves of 32 x 128
+    {256, 96, 32, 8.9, 1.33, 0.95, 0.86, 1.05, 0.65},  // eight waves of 32 x 96
+    {128, 64, 64, 8.2, 1.13, 0.37, 0.91, 1.09, 0.65},  // two wave groups of four 32 x 64
+    {128, 64, 32, 6.4, 0.67, 0.13, 0.86, 1.12, 0.0},  // four waves of 32 x 64, two workgroups a CU
+    {64, 64, 32, 5.1, 0.49, 0.03, 0.83, 1.22, 0.65},   // four waves of 16 x 64, three workgroups a CU
 };
 constexpr int kSbfNumCfgs = (int)(sizeof(kSbfCfgs) / sizeof(kSbfCfgs[0]));
 // int8 / int4 run the first two only, with these terms
-constexpr SbfCfg kSbfIntCfgs[] = {{256, 128, 32, 6.2, 0.93, 0.32, 0.0, 0.0}, {256, 96, 32, 5.1, 0.83, 0.30, 0.0, 0.0}};
+constexpr SbfCfg kSbfIntCfgs[] = {{256, 128, 32, 6.2, 0.93, 0.32, 0.0, 0.0, 0.0}, {256, 96, 32, 5.1, 0.83, 0.30, 0.0, 0.0, 0.0}};
 constexpr int kSbfNumIntCfgs = (int)(sizeof(kSbfIntCfgs) / sizeof(kSbfIntCfgs[0]));
 bool sbf_int(int fmt) { return fmt == TML_FMT_Q8_0 || fmt == TML_FMT_Q4_0; }
-int sbf_num_cfgs(int fmt) { return sbf_int(fmt) ? kSbfNumIntCfgs : kSbfNumCfgs; }
+// Int8 / int4 outside gemm_qbf.hip's layouts (odd N, K % 8 != 0, an A on no 16-byte
+// boundary), where the fp32 matrix cores' general kernel ran: at its precision.
+bool sbf_exact(const MatmulArgs &m) { return sbf_int(m.fmt) && !gemm_qbf_supported(m); }
+bool sbf_fast(const MatmulArgs &m) { return sbf_int(m.fmt) && gemm_qbf_supported(m); }
+bool sbf_cfg_ok(const MatmulArgs &m, int c) {
+    if (sbf_fast(m)) return c >= 0 && c < kSbfNumIntCfgs;
+    return c >= 0 && c < kSbfNumCfgs && (!sbf_int(m.fmt) || kSbfCfgs[c].exact > 0.0);
+}
 
 template <int FMT>
 void launch_sbf_cfg(int cfg, unsigned grid, const SbfArgs &a, hipStream_t s) {
@@ -679,6 +693,12 @@ void launch_sbf_cfg(int cfg, unsigned grid, const SbfArgs &a, hipStream_t s) {
         // two slices of loads ahead; four measured the same
         if (cfg == 0) gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 2><<<grid, 512, 0, s>>>(a);
         else gemm_sbf_kernel<FMT, 256, 96, 32, 96, 32, 1, 8, 2><<<grid, 512, 0, s>>>(a);
+    } else if constexpr (FMT >= kSbfExact) {
+        switch (cfg) {
+            case 1: gemm_sbf_kernel<FMT, 256, 96, 32, 96, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
+            case 2: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 64, 2, 8, 2><<<grid, 512, 0, s>>>(a); break;
+            default: gemm_sbf_kernel<FMT, 64, 64, 16, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
+        }
     } else {
         switch (cfg) {  // (the large tiles' registers hold one slice of loads ahead)
             case 0: gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
@@ -696,9 +716,8 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
     if (m.fmt == TML_FMT_Q4_0 && m.N % 2 != 0) return false;
     if (m.M <= kGemvMaxM || m.K <= 0) return false;
     // A's 16-byte loads need 4-byte alignment only, and a load that crosses the end
-    // of A is checked dword by dword: any K serves.  (Int8 / int4: the layouts that
-    // the kernel they compete with takes.)
-    if (sbf_int(m.fmt) ? m.K % 4 != 0 || ((uintptr_t)m.A % 16) != 0 : ((uintptr_t)m.A % 4) != 0) return false;
+    // of A is checked dword by dword: any K serves.
+    if (((uintptr_t)m.A % 4) != 0) return false;
     const uint64_t esz = m.fmt == TML_FMT_F32 ? 4 : m.fmt == TML_FMT_F16 ? 2 : 1;  // (int4: half, bounded as a byte)
     if ((uintptr_t)m.B % esz != 0) return false;
     if (m.fmt == TML_FMT_Q8_K && (m.block != 32 || m.N % 32 != 0 || ((uintptr_t)m.scales % 4) != 0)) return false;
@@ -736,7 +755,9 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 // element and does not split K.  Measured, us, that kernel / this one: f32
 // 9x4001x401 19.1 / 12.2, 60x401x399 20.6 / 15.3, 278x1340x2235 92 / 22.9,
 // 1500x1537x383 45.9 / 30.3, 2500x3001x1999 501 / 186, 30x777x4999 188 / 30.3; F16
-// 700x1111x1777 134 / 32.9, 20x3333x501 32.3 / 11.7.
+// 700x1111x1777 134 / 32.9, 20x3333x501 32.3 / 11.7; Q8_0 278x1341x2235 148 / 24.8,
+// 20x3333x501 31.5 / 11.7, per-column 2000x2999x1500 325 / 102.  2-norm error against
+// 64 bits 3.4e-7 - 1.3e-6 / 0.6e-7 - 2.8e-7.
 //
 // K is split s ways where the tiles leave CUs idle, at least eight slices a split;
 // the reduce launch costs 2.5 us and the partials' traffic, s M N 8 bytes at 6
@@ -748,13 +769,13 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 // call keeps being served under stream capture and without allocation.
 bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p) {
     constexpr double kCus = 256.0;
-    const bool is_int = sbf_int(m.fmt);
+    const bool is_int = sbf_fast(m), exact = sbf_int(m.fmt) && !is_int;
     const double mn = (double)m.M * (double)m.N;
     double best = other_us * (m.fmt == TML_FMT_F32 || is_int ? 1.1 : m.fmt == TML_FMT_Q8_K ? 0.95 : 1.0);
     int cfg = -1, nsplit = 1;
-    for (int c = 0; c < sbf_num_cfgs(m.fmt); ++c) {
+    for (int c = 0; c < (is_int ? kSbfNumIntCfgs : kSbfNumCfgs); ++c) {
         const SbfCfg &t = is_int ? kSbfIntCfgs[c] : kSbfCfgs[c];
-        const double rel = m.fmt == TML_FMT_F16 ? t.f16 : m.fmt == TML_FMT_Q8_K ? t.q8k : 1.0;
+        const double rel = m.fmt == TML_FMT_F16 ? t.f16 : m.fmt == TML_FMT_Q8_K ? t.q8k : exact ? t.exact : 1.0;
         if (rel == 0.0) continue;
         const int64_t tiles = ((m.M + t.bm - 1) / t.bm) * ((m.N + t.bn - 1) / t.bn);
         const int64_t slices = (m.K + t.bk - 1) / t.bk;
@@ -785,7 +806,7 @@ bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p
         }
     }
     const int forced = env_int("TML_GEMM_SBF_TILE", 0) - 1;
-    if (forced >= 0 && forced < sbf_num_cfgs(m.fmt)) {
+    if (sbf_cfg_ok(m, forced)) {
         cfg = forced;
         nsplit = std::max(1, env_int("TML_GEMM_SBF_SPLIT", 1));
     }
@@ -799,7 +820,7 @@ bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p
 }
 
 Status launch_gemm_sbf(const MatmulArgs &m, const GemmPlan &p, const Workspace &ws, hipStream_t s) {
-    if (!gemm_sbf_supported(m) || p.cfg < 0 || p.cfg >= sbf_num_cfgs(m.fmt))
+    if (!gemm_sbf_supported(m) || !sbf_cfg_ok(m, p.cfg))
         return Status::Err(TML_ERR_INVALID_ARG, "split-bf16 GEMM: operands or tile config not supported");
     SbfArgs a;
     a.M = (int)m.M; a.N = (int)m.N; a.K = (int)m.K;
@@ -831,8 +852,14 @@ Status launch_gemm_sbf(const MatmulArgs &m, const GemmPlan &p, const Workspace &
         case TML_FMT_F32: launch_sbf_cfg<TML_FMT_F32>(p.cfg, (unsigned)grid, a, s); break;
         case TML_FMT_F16: launch_sbf_cfg<TML_FMT_F16>(p.cfg, (unsigned)grid, a, s); break;
         case TML_FMT_Q8_K: launch_sbf_cfg<TML_FMT_Q8_K>(p.cfg, (unsigned)grid, a, s); break;
-        case TML_FMT_Q8_0: launch_sbf_cfg<TML_FMT_Q8_0>(p.cfg, (unsigned)grid, a, s); break;
-        case TML_FMT_Q4_0: launch_sbf_cfg<TML_FMT_Q4_0>(p.cfg, (unsigned)grid, a, s); break;
+        case TML_FMT_Q8_0:
+            if (sbf_exact(m)) launch_sbf_cfg<TML_FMT_Q8_0 + kSbfExact>(p.cfg, (unsigned)grid, a, s);
+            else launch_sbf_cfg<TML_FMT_Q8_0>(p.cfg, (unsigned)grid, a, s);
+            break;
+        case TML_FMT_Q4_0:
+            if (sbf_exact(m)) launch_sbf_cfg<TML_FMT_Q4_0 + kSbfExact>(p.cfg, (unsigned)grid, a, s);
+            else launch_sbf_cfg<TML_FMT_Q4_0>(p.cfg, (unsigned)grid, a, s);
+            break;
         default: return Status::Err(TML_ERR_INVALID_FORMAT, "unknown weight format");
     }
     TML_HIP_TRY(hipGetLastError());
