@@ -20,7 +20,8 @@ The same JSON line also carries:
   batches       the K timed sweeps as 5 consecutive batches (HIP events on
                 the stream the sweeps run on), each batch's TFLOP/s and
                 their median;
-  roofline      the GEMM kernel against the fp32 MFMA peak (157.3 TFLOP/s),
+  roofline      the GEMM kernel against the dense bf16 MFMA peak over the six
+                bf16 products it issues per fp32 product (417 TFLOP/s),
                 from HIP events over the timed region on the launch stream;
   config5_q     the same sweep with Q8_0 and Q4_0 weights;
   config2       the XLM-R-large layer linears at seq 512 (configs[1]);
@@ -44,6 +45,7 @@ sys.path.insert(0, ROOT)
 
 FP32_PEAK_TFLOPS = 157.3
 BF16_PEAK_TFLOPS = 2500.0  # dense bf16 MFMA
+SBF_PRODUCTS = 6  # bf16 MFMA products of an fp32 one in gemm_sbf_kernel
 HBM_PEAK_GBS = 8000.0
 
 
@@ -349,11 +351,13 @@ def main():
         per_shape[name] = {"M": M, "N": N, "K": K_, "us": round(ms * 1e3, 2),
                            "tflops": round(2.0 * M * N * K_ / ms / 1e9, 2)}
     achieved = sweep_flops / (ev_ms / K) / 1e9
-    roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "frac": round(achieved / FP32_PEAK_TFLOPS, 4), "traffic": traffic_per_sweep(),
+    peak = BF16_PEAK_TFLOPS / SBF_PRODUCTS
+    roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": round(peak, 1), "unit": "TFLOP/s",
+                "frac": round(achieved / peak, 4), "frac_of_fp32_mfma_peak": round(achieved / FP32_PEAK_TFLOPS, 4),
+                "traffic": traffic_per_sweep(),
                 "algorithmic_bytes": int(L * sum(4 * (M * K_ + K_ * N + M * N) for (_, M, N, K_) in ENC_SHAPES)),
-                "kernel": "gemm_dma_kernel<f32 B> (128x64 tiles, 8 waves, BK 32, three LDS stages; FFN-down K "
-                          "split 2 + splitk_reduce_kernel), v_mfma_f32_16x16x4_f32",
+                "kernel": "gemm_sbf_kernel<f32> (three-term bf16 splits, tiles and K splits of pick_sbf), "
+                          "v_mfma_f32_16x16x32_bf16",
                 "per_unit": "2*M*N*K flop per GEMM launch; 96 launches per sweep",
                 "per_shape": per_shape}
     log(f"roofline: {json.dumps(roofline)}")
@@ -406,7 +410,7 @@ def main():
 def traffic_per_sweep():
     """HBM bytes per headline sweep from the committed rocprofv3 PMC summary
     (FETCH_SIZE + WRITE_SIZE per dispatch, scaled by a plain copy kernel),
-    or None when the summary is absent."""
+    or None when the summary is absent or of another kernel."""
     path = os.path.join(ROOT, "profiles", "gemm_whisper_encoder_traffic.json")
     try:
         with open(path) as f:
