@@ -150,10 +150,10 @@ int tml_hip_sgemm_q8(int64_t M, int64_t N, int64_t K, const float *A, const int8
  * faster, the larger products -- the bf16 matrix cores with every operand split
  * exactly into bf16 terms and the products of the terms summed in fp32, dropped
  * terms below 2^-25 of a product; both are fp32 results (2-norm error against 64
- * bits 1e-7 to 1e-6).  Infinities, NaNs, values past the largest bf16 and sums
- * below 2^-70 are recomputed as ascending fp32 sums.  Limit: where one operand
- * is past 2^22 in magnitude, the other's elements below 2^-109 are taken to an
- * absolute 2^-134. */
+ * bits 1e-7 to 1e-6).  Outputs that the terms cannot carry -- infinities, NaNs,
+ * operands past the largest bf16, sums (zero included) that an operand below 2^-102
+ * or a product below 2^-80 may have put off by 2^-24 of themselves -- are recomputed from the operands
+ * in fp32. */
 
 /* C = A . dequant(Q8_K B).  Replaces zblas.sgemmQ8K(m, n, k, a, b.data,
  * b.scales, b.block_size, c) at src/core/quantization.zig:555

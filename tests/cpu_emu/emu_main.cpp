@@ -18,7 +18,7 @@
 //                   device and dequantized (errors are expected for most)
 //   flags  any of: b bias, r residual, e GELU (erf), t GELU (tanh), B beta != 0; "-" for none;
 //          S allocates B 16 bytes short of its size (a planted mistake: the
-//          harness must report it)
+//          harness must report it); N makes the bf16 matrix cores return NaN
 //   NAME=VALUE  environment for this case only (the library's tuning overrides)
 // Output: "ok <line>" or "err <code> <message> <line>" per case; exit 0.
 #include <cstdint>
@@ -196,6 +196,7 @@ int main() {
         std::fprintf(stdout, "run %s\n", line.c_str());
         std::fflush(stdout);
         const long long launches0 = tml_emu_launches;
+        tml_emu_mfma_nan = op != "tlfile" && flags.find('N') != std::string::npos;
         const int rc = run_case(op, fmt, M, N, K, flags);
         for (auto &kv : env) unsetenv(kv.substr(0, kv.find('=')).c_str());
         if (rc == 0)

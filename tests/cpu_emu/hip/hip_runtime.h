@@ -18,10 +18,12 @@
 //
 // What is NOT emulated: cross-lane data (DPP, swizzles and shuffles return
 // the lane's own value), the contents other threads leave in LDS, and the
-// matrix-core arithmetic.  Results are therefore meaningless; only the
+// matrix-core arithmetic (the sums stay zero, or become NaN where a case asks for
+// it).  Results are therefore meaningless; only the
 // addresses are checked.  Control flow depends on the arguments only
 // (plus the split-K arrival counters, which behave as on the device when
-// the blocks run one after another).
+// the blocks run one after another, and the split-bf16 GEMM's second look at
+// sums that are zero or NaN).
 #pragma once
 
 #include <algorithm>
@@ -232,6 +234,7 @@ tml_emu_launcher<P...> tml_emu_launch(void (*k)(P...), dim3 g, dim3 b, size_t sh
 // ------------------------------------------------------------- device side
 inline void __syncthreads() {}
 inline int __syncthreads_or(int v) { return v; }
+inline int __any(int v) { return v; }
 template <typename A, typename B>
 inline std::common_type_t<A, B> min(A a, B b) {
     return a < b ? a : b;
@@ -282,10 +285,12 @@ template <typename T>
 inline T __builtin_amdgcn_readfirstlane(T v) {
     return v;
 }
+inline bool tml_emu_mfma_nan = false;  // the bf16 matrix cores' sums are NaN
 inline tml_emu_f32x4 __builtin_amdgcn_mfma_f32_16x16x4f32(float, float, tml_emu_f32x4 c, int, int, int) { return c; }
 typedef __bf16 tml_emu_bf16x8 __attribute__((ext_vector_type(8)));
 inline tml_emu_f32x4 __builtin_amdgcn_mfma_f32_16x16x32_bf16(tml_emu_bf16x8, tml_emu_bf16x8, tml_emu_f32x4 c, int, int,
                                                             int) {
+    if (tml_emu_mfma_nan) c = tml_emu_f32x4{NAN, NAN, NAN, NAN};
     return c;
 }
 inline float __builtin_amdgcn_fmed3f(float a, float b, float c) { return a < b ? b : (a > c ? c : a); }

@@ -363,3 +363,18 @@ def test_sbf_cases(emu):
     for fmt in (F32, F16, Q8_K):
         _, fails = run_cases(emu, [f"gemm {fmt} 200 352 512 S TML_GEMM_SBF_TILE=2"], workers=1)
         assert fails, f"the CPU build did not report a short operand of format {fmt}"
+
+
+def test_sbf_second_look(emu):
+    # outputs the split does not carry (gemm_sbf.hip, sbf_repair): the rows of A and
+    # columns of B read again for zero and for NaN sums, every format, tile and K split,
+    # on shapes ragged in M, N and K
+    cases = []
+    for tile in range(1, 6):
+        for fmt, n in [(F32, 131), (F16, 131), (Q8_K, 160)] + ([(Q8_0, 131), (Q4_0, 130)] if tile in (2, 3, 5) else []) + \
+                ([(Q8_0, 136), (Q4_0, 130)] if tile <= 2 else []):
+            for flags, k in (("b", 72), ("N", 72), ("N", 101)):
+                for split in (1, 2):
+                    cases.append(f"gemm {fmt} 140 {n} {k} {flags} TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT={split}")
+    outs, fails = run_cases(emu, cases)
+    assert not fails and not _err_lines(outs), (fails, _err_lines(outs)[:3])

@@ -6,10 +6,10 @@ of the same operands by at most one fp32 rounding of each 32-deep slice's sum,
 the six dropped or merged small terms (below 2^-24 of a product together) and
 the epilogue's own roundings:
     |C - ref| <= (ceil(K / 32) + 8) * 2^-24 * sum_k |a b| + 2^-23 |ref|.
-Operands the split does not carry (infinities, NaNs, values past the largest
-bf16, sums of products below 2^-70) are recomputed in fp32 in ascending k, as
-the reference does (src/core/ops.zig:277-414), so their inf / NaN pattern is the
-oracle's.  Int8 / int4 weights take two terms of A (|x - hi - lo| <= 2^-17 |x|) and
+Outputs the split does not carry (infinities, NaNs, values past the largest
+bf16, sums that elements below 2^-102 or products below 2^-80 may have put off) are
+recomputed in fp32, as the reference sums (src/core/ops.zig:277-414), so their inf /
+NaN pattern is the oracle's.  Int8 / int4 weights take two terms of A (|x - hi - lo| <= 2^-17 |x|) and
 share one sum, which a slice rounds twice:
     |C - ref| <= (2^-17 + (2 ceil(K / 32) + 8) * 2^-24) * sum_k |a b| + 2^-23 |ref|.
 A K split adds one rounding a split.  TML_GEMM_SBF_TILE / _SPLIT pick a tile and
@@ -152,6 +152,51 @@ def test_sbf_range(env, scale):
     ref = a.astype(np.float64) @ w.astype(np.float64)
     mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64)
     assert np.max(np.abs(c - ref) / mag) <= k * 2.0**-24
+
+
+SMALL = [(-115, 60), (-120, 60), (-125, 70), (-130, 90), (-135, 21), (-140, 100), (60, -120), (90, -130), (100, -140)]
+
+
+@pytest.mark.parametrize("tile,split", [(t, 1) for t in TILES] + [(3, 2), (5, 3)])
+@pytest.mark.parametrize("ea,eb", SMALL)
+def test_sbf_small_operands(env, tile, split, ea, eb):
+    """Operands whose terms reach bf16's denormals, or have none (below 2^-134),
+    against large ones: fp32 precision, K roundings at most, as the fp32 matrix cores give."""
+    env["TML_GEMM_SBF_TILE"], env["TML_GEMM_SBF_SPLIT"] = str(tile), str(split)
+    m, n, k = 140, 101, 130
+    a, w = np.ldexp(synth.normal_matrix(101, m, k), ea), np.ldexp(synth.normal_matrix(102, k, n), eb)
+    a[7] = 0.0  # a sum of zeros
+    w[:, 9] = 0.0
+    a[11, 1::2], w[1::2, 12] = -a[11, ::2], w[::2, 12]  # and of values that cancel
+    # row 70 tiny among ordinary values, one large column: only their own outputs are in doubt
+    a[70], w[:, 70] = np.ldexp(a[70], -ea - 125), np.ldexp(w[:, 70], 20 - eb)  # (2^20: the large products stay finite)
+    c = run(_abi.FMT_F32, m, n, k, a, w, None).astype(np.float64)
+    ref = a.astype(np.float64) @ w.astype(np.float64)
+    mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64)
+    # (2^-149 a product where the fp32 products themselves are denormal)
+    bound = k * 2.0**-24 * mag + np.where(mag < 2.0**-100, k * 2.0**-149, 0.0)
+    assert np.all(np.abs(c - ref) <= bound), float(np.max(np.abs(c - ref) / (mag + 1e-300)))
+
+
+@pytest.mark.parametrize("tile", [2, 3, 5])
+@pytest.mark.parametrize("fmt,ea,ew", [(_abi.FMT_F16, -138, 12), (_abi.FMT_Q8_K, -125, 60), (_abi.FMT_Q8_K, 90, -130),
+                                       (_abi.FMT_Q8_0, -138, 0)])
+def test_sbf_small_operands_formats(orc, env, tile, fmt, ea, ew):
+    # the same with f16, Q8_K and (odd N: three terms) int8 weights
+    env["TML_GEMM_SBF_TILE"] = str(tile)
+    m, n, k = 140, 96 if fmt == _abi.FMT_Q8_K else 97, 130
+    a, scale = np.ldexp(synth.normal_matrix(103, m, k), ea), 1.0
+    raw = synth.normal_matrix(104, k, n)
+    if fmt == _abi.FMT_Q8_0:
+        (q, _), scales, scale = orc.quantize_q8(raw), None, 2.0**20
+        w = q.reshape(k, n).astype(np.float64) * scale
+    else:
+        q, scales, w = weight(orc, fmt, np.ldexp(raw, ew))
+    c = np.zeros((m, n), np.float32)
+    _abi.gemm(fmt, m, n, k, a, np.ascontiguousarray(q), c, scale=scale, scales=scales)
+    ref = a.astype(np.float64) @ w.astype(np.float64)
+    mag = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64)
+    assert np.all(np.abs(c - ref) <= k * 2.0**-24 * mag), float(np.max(np.abs(c - ref) / mag))
 
 
 def test_sbf_exact_integers(env):

@@ -30,11 +30,16 @@
 // two products take a third of the matrix-core time, and LDS and the loads' issue
 // are as large.
 //
-// Values the split does not carry -- infinities and NaNs (their residual is
-// NaN), |x| above the largest bf16, and magnitudes so small that l falls under
-// bf16's denormals (|x| < 2^-109) -- show in the sum: it is not finite, or not
-// zero and below 2^-70.  The epilogue recomputes such an output from the
-// operands as an ascending fp32 sum, the reference's own.
+// Values the split does not carry.  Infinities, NaNs (their residual is NaN) and
+// |x| above the largest bf16 make the sum infinite or NaN.  Of a nonzero |x| < 2^-102
+// up to 2^-124 may be lost (its terms reach bf16's denormals; the largest value
+// below 2^-134 has none at all), so a sum of K products is off by up to K 2^-124 times
+// the largest of the other operand, and by K 2^-122 where products of terms
+// themselves fall below 2^-126.  An output smaller than 2^24 times what it may be off by
+// -- zero included -- is recomputed from the operands (sbf_repair), as is one that
+// is not finite.  The split notes the largest magnitude that passes through it (one
+// v_max3 a pair of values, 11 instructions before), so outputs of 2^-70 and more need no second look
+// unless an operand is past 2^28 / K.
 #include "tml_internal.hpp"
 
 #include <algorithm>
@@ -133,17 +138,127 @@ __device__ __forceinline__ float sbf_b(const SbfArgs &a, int k, int n) {
     else return (float)((const int8_t *)a.B)[(size_t)k * a.N + n] * a.scales[((size_t)k * a.N + n) >> 5];
 }
 
-// A sum that shows operands the split does not carry (top of the file).
-__device__ __forceinline__ bool sbf_suspect(float v) {
-    const uint32_t u = __float_as_uint(v) & 0x7FFFFFFFu;
-    return u - 1u >= 0x7F7FFFFFu || u - 1u < 0x1C7FFFFFu ? u != 0u : false;  // not finite, or 0 < |v| < 2^-70
-}
+__device__ __forceinline__ bool sbf_not_finite(float v) { return (__float_as_uint(v) & 0x7F800000u) == 0x7F800000u; }
+// The magnitude B cannot exceed; 0 where the split has to note it.
+template <int FMT>
+constexpr float kSbfTopB = FMT == TML_FMT_F16 ? 65504.0f : kSbfPlanesB<FMT> == 3 ? 0.0f : 128.0f;
+// Below this an output may be off by more than 2^-24 of itself, where no operand of its
+// tile exceeds top and kk products are summed (top of the file).
+__device__ __forceinline__ float sbf_doubt(float kk, float top) { return kk * 0x1p-98f + kk * 0x1p-99f * top; }
 // The ascending fp32 sum of output (row, col)'s products over k in [k0, k1).
 template <int FMT>
 __device__ __forceinline__ float sbf_fp32_sum(const SbfArgs &a, int row, int col, int k0, int k1) {
     float s = 0.0f;
     for (int k = k0; k < k1; ++k) s = fmaf(a.A[(size_t)row * a.K + k], sbf_b<FMT>(a, k, col), s);
     return s;
+}
+
+// The smallest nonzero and the largest magnitude of what it has seen, as bits.
+struct SbfRange {
+    uint32_t lo = ~0u, hi = 0u;  // lo: 2 * bits - 1, so that zeros come last
+    __device__ __forceinline__ void see(float v) {
+        const uint32_t u = __float_as_uint(v);
+        lo = min(lo, (u << 1) - 1u);
+        hi = max(hi, u & 0x7FFFFFFFu);
+    }
+    __device__ __forceinline__ void see(SbfRange r) {
+        lo = min(lo, r.lo);
+        hi = max(hi, r.hi);
+    }
+    // infinity where all were zero
+    __device__ __forceinline__ float least() const {
+        return lo == ~0u ? __builtin_huge_valf() : __uint_as_float((lo + 1u) >> 1);
+    }
+    __device__ __forceinline__ float most() const { return __uint_as_float(hi); }
+};
+
+// Puts right the outputs in ct, the tile's sums over k in [kbase, kend), that the split
+// does not carry (top of the file).  Small ones are first weighed by what their own
+// row of A and column of B hold: a sum of zeros, or of values that cancel, is as good as
+// any, and rows of zeros are told apart before any column is read.  top: the
+// largest magnitude this lane has split.  ex: LDS, sbf_repair_floats floats.
+template <int BM, int BN, int NW>
+constexpr int kSbfRepairFloats = 2 * (BM + 64 * NW);
+template <int FMT, int BM, int BN, int NW>
+__device__ __forceinline__ void sbf_repair(const SbfArgs &a, float *ct, float *ex, float top, int m0, int n0, int kbase,
+                                           int kend) {
+    constexpr int NT = 64 * NW, CS = BN + 4, G = NT / BN;
+    int tid = threadIdx.x;
+    __asm__ volatile("" : "+v"(tid));  // (nothing of this is computed before the K loop and held through it)
+    const int lane = tid & 63, wave = tid >> 6;
+    const int rows = min(BM, a.M - m0), cols = min(BN, a.N - n0);
+    const float kk = (float)(kend - kbase);
+    SbfRange *const rrow = (SbfRange *)ex, *const rcol = rrow + BM;
+    if constexpr (kSbfTopB<FMT> == 0.0f) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+        if (lane == 0) ex[wave] = top;
+        __syncthreads();
+        for (int w = 0; w < NW; ++w) top = fmaxf(top, ex[w]);
+    }
+    const float doubt = sbf_doubt(kk, top);
+    int small = 0;
+#pragma unroll 4
+    for (int e = tid; e < BM * BN; e += NT)
+        small |= e / BN < rows && e % BN < cols && fabsf(ct[e / BN * CS + e % BN]) < doubt;
+    if (__syncthreads_or(small)) {
+        for (int r = wave; r < rows; r += NW) {
+            int any = 0;
+            for (int n = lane; n < cols; n += 64) any |= fabsf(ct[r * CS + n]) < doubt;
+            if (!__any(any)) continue;
+            const float *const row = a.A + (size_t)(m0 + r) * a.K;
+            SbfRange x;
+#pragma unroll 8
+            for (int k = kbase + lane; k < kend; k += 64) x.see(row[k]);
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                SbfRange y;
+                y.lo = (uint32_t)__shfl_xor((int)x.lo, o);
+                y.hi = (uint32_t)__shfl_xor((int)x.hi, o);
+                x.see(y);
+            }
+            if (lane == 0) rrow[r] = x;
+        }
+        __syncthreads();
+        small = 0;
+        for (int e = tid; e < BM * BN; e += NT)
+            small |= e / BN < rows && e % BN < cols && fabsf(ct[e / BN * CS + e % BN]) < doubt && rrow[e / BN].lo != ~0u;
+        if (__syncthreads_or(small)) {
+            const int n = tid % BN, grp = tid / BN;
+            if (grp < G) {
+                SbfRange x;
+                if (n < cols) {
+#pragma unroll 8
+                    for (int k = kbase + grp; k < kend; k += G) x.see(sbf_b<FMT>(a, k, n0 + n));
+                }
+                rcol[tid] = x;
+            }
+            __syncthreads();
+            if (tid < BN) {
+                for (int z = 1; z < G; ++z) rcol[tid].see(rcol[tid + z * BN]);
+            }
+            __syncthreads();
+            for (int e = tid; e < BM * BN; e += NT) {
+                const int r = e / BN, c = e % BN;
+                float *const v = &ct[r * CS + c];
+                if (r >= rows || c >= cols || !(fabsf(*v) < doubt)) continue;
+                const SbfRange x = rrow[r], y = rcol[c];
+                if (x.lo == ~0u || y.lo == ~0u) continue;  // a sum of zeros
+                float off = x.least() * y.least() < 0x1p-80f ? kk * 0x1p-98f : 0.0f;  // (2^-23 twice down to the last bits' product)
+                if (x.least() < 0x1p-102f) off += kk * 0x1p-100f * y.most();
+                if (y.least() < 0x1p-102f) off += kk * 0x1p-100f * x.most();
+                if (fabsf(*v) < off) *v = __builtin_nanf("");
+            }
+            __syncthreads();
+        }
+    }
+#pragma unroll 1
+    for (int e = tid; e < BM * BN; e += NT) {
+        const int r = e / BN, c = e % BN;
+        float *const v = &ct[r * CS + c];
+        if (r < rows && c < cols && sbf_not_finite(*v)) *v = sbf_fp32_sum<FMT>(a, m0 + r, n0 + c, kbase, kend);
+    }
+    __syncthreads();
 }
 
 // A workgroup of NW = 4 or 8 waves owns a BM x BN tile of C, each wave a WM x
@@ -187,7 +302,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     constexpr int CS = BN + 4;            // floats of a staged C row (rows 4 apart: 16 banks on)
     constexpr int kARows = 3 * kStage;    // AL: the waves' own A rows, WM x 8 slots each
     constexpr int kLoop = kARows + (AL ? NW * WM * 8 : 0);
-    constexpr int kLds = kLoop > BM * CS / 4 ? kLoop : BM * CS / 4;
+    constexpr int kTile = (BM * CS + kSbfRepairFloats<BM, BN, NW>) / 4;  // the epilogue's
+    constexpr int kLds = kLoop > kTile ? kLoop : kTile;
     __shared__ uintx4 lds[kLds];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -303,17 +419,25 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 
     // ---- splitting, a pair of k at a time: A's pair e to word e of the next
     // slice's operands, B's to word e of the slots write_b stores.
+    constexpr bool TOP = kSbfTopB<FMT> == 0.0f;
+    float top = kSbfTopB<FMT>;  // the largest magnitude split
+    auto note = [&](float x, float y) __attribute__((always_inline)) {
+        if constexpr (TOP) top = fmaxf(fmaxf(top, fabsf(x)), fabsf(y));
+    };
     uintx4 av[2][NA][TM], bp[PB][NB];
+    float bx[PB][4][2];  // B's values, for note()
     auto split_a = [&](int i, int e, int d, int nxt) __attribute__((always_inline)) {
         uint32_t t[NA];
-        sbf_split<NA>(__uint_as_float(AL ? rr[i][2 * e] : ra[d][i][2 * e]),
-                      __uint_as_float(AL ? rr[i][2 * e + 1] : ra[d][i][2 * e + 1]), t);
+        const float x = __uint_as_float(AL ? rr[i][2 * e] : ra[d][i][2 * e]);
+        const float y = __uint_as_float(AL ? rr[i][2 * e + 1] : ra[d][i][2 * e + 1]);
+        note(x, y);
+        sbf_split<NA>(x, y, t);
 #pragma unroll
         for (int p = 0; p < NA; ++p) av[nxt][p][i][e] = t[p];
     };
     auto split_b = [&](int t, int e, int d) __attribute__((always_inline)) {
 #pragma clang fp contract(off)  // (the dequantized value is the rounded product, in every tile)
-        float x[2];
+        float *const x = bx[t][e];
 #pragma unroll
         for (int z = 0; z < 2; ++z) {
             const uint32_t w = rb[d][t][2 * e + z];
@@ -329,7 +453,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         for (int p = 0; p < NB; ++p) bp[t][p][e] = v[p];
     };
     auto write_b = [&](int t, int p, int stage) __attribute__((always_inline)) {
-        if (TB % NT == 0 || tid + t * NT < TB) lds[stage + slot_b[t] + p * BN * SL] = bp[t][p];
+        if (TB % NT == 0 || tid + t * NT < TB) {
+            lds[stage + slot_b[t] + p * BN * SL] = bp[t][p];
+            if (p == 0) {  // (here, so that threads without a task split nothing: noted in split_b, 9-16 registers more)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) note(bx[t][e][0], bx[t][e][1]);
+            }
+        }
     };
 
     // acc holds the hh products, cor the five (four) smaller ones: a slice
@@ -544,37 +674,39 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // activation in every element it cost 36 k cycles a tile (16 of the 102 us of
     // 1500x5120x1280).
     float *const ct = (float *)lds;
-    int suspect = 0;
+    // not finite, or below `least` (no less than sbf_doubt, top permitting); of the
+    // rows and columns past the matrix, whose sums are zeros, none is looked at
+    const float kk = (float)(kend - kbase), least = fmaxf(0x1p-70f, sbf_doubt(kk, kSbfTopB<FMT>));
+    const uint32_t least_u = __float_as_uint(least);
+    uint32_t worst = 0;
     auto put = [&](bool add) __attribute__((always_inline)) {
+        const int rows = a.M - m0 - wm0 - 4 * g, cols = a.N - n0 - wn0 - c;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+            for (int e = 0; e < 4; ++e) {
+                uint32_t w = 0;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
+                for (int j = 0; j < TN; ++j) {
                     float *const to = &ct[(wm0 + 16 * i + 4 * g + e) * CS + wn0 + 16 * j + c];
                     const float v = add ? *to + acc[i][j][e] : acc[i][j][e];
-                    suspect |= sbf_suspect(v);
+                    w = max(w, 16 * j < cols ? (__float_as_uint(v) & 0x7FFFFFFFu) - least_u : 0u);
                     *to = v;
                 }
+                worst = max(worst, 16 * i + e < rows ? w : 0u);
+            }
     };
     if constexpr (KW == 1) {
         put(false);
     } else {
         if (kg == 1) put(false);
-        suspect = 0;
+        worst = 0;
         __syncthreads();
         if (kg == 0) put(true);
     }
-    if (__syncthreads_or(suspect)) {
-#pragma unroll 1
-        for (int e = tid; e < BM * BN; e += NT) {
-            const int tr = e / BN, row = m0 + tr, col = n0 + e % BN;
-            float *const v = &ct[tr * CS + e % BN];
-            if (row < a.M && col < a.N && sbf_suspect(*v)) *v = sbf_fp32_sum<FMT>(a, row, col, kbase, kend);
-        }
-        __syncthreads();
-    }
+    const bool suspect = worst >= 0x7F800000u - least_u || (TOP && top > 0x1p28f / kk);
+    if (__syncthreads_or(suspect))
+        sbf_repair<FMT, BM, BN, NW>(a, ct, ct + BM * CS, top, m0, n0, kbase, kend);
     constexpr int CH = BN / 4, RPP = NT / CH;  // 16-byte pieces of a tile row; rows a pass
     const int pc = 4 * (tid % CH), tr0 = tid / CH, col = n0 + pc;  // a thread's pieces lie in one column of pieces
     if (tr0 >= RPP || col >= a.N) return;
