@@ -152,8 +152,9 @@ int tml_hip_sgemm_q8(int64_t M, int64_t N, int64_t K, const float *A, const int8
  * terms below 2^-25 of a product; both are fp32 results (2-norm error against 64
  * bits 1e-7 to 1e-6).  Outputs that the terms cannot carry -- infinities, NaNs,
  * operands past the largest bf16, sums (zero included) that an operand below 2^-102
- * or a product below 2^-80 may have put off by 2^-24 of themselves -- are recomputed from the operands
- * in fp32. */
+ * or a product below 2^-80 may have put off by 2^-24 of themselves -- are
+ * recomputed from the operands on the fp32 matrix cores, at most five times the time of
+ * a call with none. */
 
 /* C = A . dequant(Q8_K B).  Replaces zblas.sgemmQ8K(m, n, k, a, b.data,
  * b.scales, b.block_size, c) at src/core/quantization.zig:555

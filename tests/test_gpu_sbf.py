@@ -280,6 +280,47 @@ def test_sbf_int_inf_nan(orc, env, tile):
     assert np.all(np.abs(c[fin].astype(np.float64) - ref[fin]) <= (2.0**-17 + 2.0**-23 * k) * mag[fin])
 
 
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("fmt,n,k,tile", [(_abi.FMT_F32, 101, 101, 1), (_abi.FMT_F32, 101, 101, 4), (_abi.FMT_F16, 101, 101, 2),
+                                          (_abi.FMT_F16, 101, 101, 5), (_abi.FMT_Q8_K, 160, 101, 2),
+                                          (_abi.FMT_Q8_K, 160, 101, 3), (_abi.FMT_Q8_0, 104, 136, 1),
+                                          (_abi.FMT_Q4_0, 98, 136, 1), (_abi.FMT_Q4_0, 98, 136, 2),
+                                          (_abi.FMT_Q8_0, 101, 101, 2), (_abi.FMT_Q8_0, 101, 101, 5),
+                                          (_abi.FMT_Q4_0, 98, 101, 3)])
+def test_sbf_recomputed(orc, env, fmt, n, k, tile, split):
+    # rows, columns and single elements that are not finite, every format on both
+    # its arithmetics (k = 136: two terms of A, n odd or k = 101: three), with and without a
+    # K split: the 64-bit product's pattern, and fp32 sums of K products elsewhere
+    env["TML_GEMM_SBF_TILE"], env["TML_GEMM_SBF_SPLIT"] = str(tile), str(split)
+    m, scale, scales = 140, 1.0, None
+    a, raw = synth.normal_matrix(111, m, k), synth.normal_matrix(112, k, n, 0.02)
+    a[3, 5], a[4, 0], a[31, 70], a[64, k - 1], a[90], a[139, 7] = np.inf, -np.inf, np.nan, np.inf, np.nan, np.inf
+    raw[5, ::7], raw[70, 1::5] = 0.0, 0.0
+    if fmt == _abi.FMT_F32:
+        raw[11, 20], raw[12, 21], raw[:, 40] = np.inf, np.nan, -np.inf
+    if fmt == _abi.FMT_Q8_0:
+        (q, scale), terms = orc.quantize_q8(raw), 2 if k % 8 == 0 and n % 8 == 0 else 3
+        w = orc.dequantize_q8(q, scale).reshape(k, n)
+    elif fmt == _abi.FMT_Q4_0:
+        (q, scale), terms = orc.quantize_q4(raw), 2 if k % 8 == 0 else 3
+        w = orc.dequantize_q4(q, k * n, scale).reshape(k, n)
+    else:
+        (q, scales, w), terms = weight(orc, fmt, raw), 3
+    if fmt == _abi.FMT_Q8_K:
+        scales = scales.copy()
+        scales[5 * n // 32 + 1] = np.nan  # 32 elements of row 5
+        w[5, 32:64] = np.nan
+    c = np.zeros((m, n), np.float32)
+    _abi.gemm(fmt, m, n, k, a, np.ascontiguousarray(q), c, scale=scale, scales=scales)
+    with np.errstate(invalid="ignore"):
+        ref = a.astype(np.float64) @ w.astype(np.float64)
+        assert np.array_equal(np.isnan(c), np.isnan(ref))
+        assert np.array_equal(np.isposinf(c), np.isposinf(ref)) and np.array_equal(np.isneginf(c), np.isneginf(ref))
+    fin, zero = np.isfinite(ref), lambda x: np.where(np.isfinite(x), np.abs(x), 0).astype(np.float64)
+    bound = (k * 2.0**-24 + (2.0**-17 if terms == 2 else 0.0)) * (zero(a) @ zero(w)) + 2.0**-22 * np.abs(np.where(fin, ref, 0))
+    assert np.all(np.abs(c - np.where(fin, ref, 0))[fin] <= bound[fin])
+
+
 def test_sbf_split_plan_without_workspace(env):
     """512 x 1024 x 4096 in f32 splits K by default; a first call under stream
     capture, where the workspace cannot grow, runs an unsplit plan instead of

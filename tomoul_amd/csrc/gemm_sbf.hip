@@ -116,6 +116,8 @@ constexpr int kSbfExact = 64;
 template <int FMT>
 constexpr int kSbfStored = FMT & ~kSbfExact;  // B's format in memory
 template <int FMT>
+constexpr unsigned kSbfBytes = FMT == TML_FMT_F32 ? 4u : FMT == TML_FMT_F16 ? 2u : 1u;  // an element's (int4: half)
+template <int FMT>
 constexpr bool kSbfInt = FMT == TML_FMT_Q8_0 || FMT == TML_FMT_Q4_0;
 template <int FMT>
 constexpr int kSbfPlanesA = kSbfInt<FMT> ? 2 : 3;
@@ -145,12 +147,73 @@ constexpr float kSbfTopB = FMT == TML_FMT_F16 ? 65504.0f : kSbfPlanesB<FMT> == 3
 // Below this an output may be off by more than 2^-24 of itself, where no operand of its
 // tile exceeds top and kk products are summed (top of the file).
 __device__ __forceinline__ float sbf_doubt(float kk, float top) { return kk * 0x1p-98f + kk * 0x1p-99f * top; }
-// The ascending fp32 sum of output (row, col)'s products over k in [k0, k1).
-template <int FMT>
-__device__ __forceinline__ float sbf_fp32_sum(const SbfArgs &a, int row, int col, int k0, int k1) {
-    float s = 0.0f;
-    for (int k = k0; k < k1; ++k) s = fmaf(a.A[(size_t)row * a.K + k], sbf_b<FMT>(a, k, col), s);
-    return s;
+
+// Recomputes the outputs of a 32 x 16 block that are not finite, on the fp32 matrix
+// cores and straight from global memory: one wave, rows row0.. of A and columns col0..
+// of B (`rows` and `cols` of them in the matrix), v the block in the staged tile.  A
+// lane's 16-byte load of A holds k = 4 g .. 4 g + 3 of a 16-deep step, and
+// matrix instruction e multiplies element e of every lane.  Bound: the fp32 matrix
+// cores and the loads' issue where a whole tile is recomputed, the loads' latency where
+// a row or column is.  1500x5120x1280 (92 us on ordinary values, 160 - 190 on the fp32-MFMA
+// kernels): every output NaN 419 us, one row 152, one column 150; with one
+// thread an output, all of K in a row, 10.3 ms, 396 us and 8.8 ms.
+// U: steps in flight.
+template <int FMT, int CS, int U>
+__device__ __forceinline__ void sbf_recompute(const SbfArgs &a, float *v, int row0, int col0, int rows, int cols,
+                                              int kbase, int kend) {
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    int bad = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int r = 16 * (e / 4) + 4 * g + e % 4;
+        bad |= r < rows && c < cols && sbf_not_finite(v[r * CS + c]);
+    }
+    if (!__any(bad)) return;
+    const __amdgpu_buffer_rsrc_t rsa = sbf_rsrc(a.A, a.a_bytes), rsb = sbf_rsrc(a.B, (unsigned)kend * (unsigned)a.ldb);
+    const __amdgpu_buffer_rsrc_t rss = sbf_rsrc(FMT == TML_FMT_Q8_K ? (const void *)a.scales : a.B, a.s_bytes);
+    const unsigned col = (unsigned)(col0 + c);
+    const unsigned b_col = kSbfStored<FMT> == TML_FMT_Q4_0 ? col / 2u : col * kSbfBytes<FMT>;
+    floatx4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll 1
+    for (int kb = kbase; kb < kend; kb += 16 * U) {
+        const int k0 = kb + 4 * g;
+        uintx4 x[U][2];
+        float y[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                x[u][t] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rsa, ((unsigned)(row0 + 16 * t + c) * (unsigned)a.K + (unsigned)(k0 + 16 * u)) * 4u, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const unsigned k = (unsigned)(k0 + 16 * u + e), off = k * (unsigned)a.ldb + b_col;  // (past kend: zero)
+                if constexpr (FMT == TML_FMT_F32) y[u][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsb, off, 0, 0));
+                else if constexpr (FMT == TML_FMT_F16) y[u][e] = tml_half_bits(__builtin_amdgcn_raw_buffer_load_b16(rsb, off, 0, 0));
+                else if constexpr (kSbfStored<FMT> == TML_FMT_Q4_0) y[u][e] = sbf_int4(__builtin_amdgcn_raw_buffer_load_b8(rsb, off, 0, 0), (int)col);
+                else y[u][e] = (float)(int8_t)__builtin_amdgcn_raw_buffer_load_b8(rsb, off, 0, 0);
+                if constexpr (FMT == TML_FMT_Q8_K)
+                    y[u][e] *= __uint_as_float(
+                        __builtin_amdgcn_raw_buffer_load_b32(rss, k * ((unsigned)a.N / 8u) + col / 32u * 4u, 0, 0));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const bool in = k0 + 16 * u + e < kend;  // (A reads on past kend)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? __uint_as_float(x[u][t][e]) : 0.0f,
+                                                                  in ? y[u][e] : 0.0f, acc[t], 0, 0, 0);
+                }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int r = 16 * (e / 4) + 4 * g + e % 4;
+        float *const to = &v[r * CS + c];
+        if (r < rows && c < cols && sbf_not_finite(*to)) *to = acc[e / 4][e % 4];
+    }
 }
 
 // The smallest nonzero and the largest magnitude of what it has seen, as bits.
@@ -183,9 +246,10 @@ template <int FMT, int BM, int BN, int NW>
 __device__ __forceinline__ void sbf_repair(const SbfArgs &a, float *ct, float *ex, float top, int m0, int n0, int kbase,
                                            int kend) {
     constexpr int NT = 64 * NW, CS = BN + 4, G = NT / BN;
+    constexpr int U = NW == 8 && FMT != TML_FMT_Q8_K ? 8 : 4;  // (no more registers than the K loop's)
     int tid = threadIdx.x;
     __asm__ volatile("" : "+v"(tid));  // (nothing of this is computed before the K loop and held through it)
-    const int lane = tid & 63, wave = tid >> 6;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rows = min(BM, a.M - m0), cols = min(BN, a.N - n0);
     const float kk = (float)(kend - kbase);
     SbfRange *const rrow = (SbfRange *)ex, *const rcol = rrow + BM;
@@ -202,22 +266,36 @@ __device__ __forceinline__ void sbf_repair(const SbfArgs &a, float *ct, float *e
     for (int e = tid; e < BM * BN; e += NT)
         small |= e / BN < rows && e % BN < cols && fabsf(ct[e / BN * CS + e % BN]) < doubt;
     if (__syncthreads_or(small)) {
-        for (int r = wave; r < rows; r += NW) {
+        // eight rows at a time, a 128-byte piece of each an instruction
+        const __amdgpu_buffer_rsrc_t rsa = sbf_rsrc(a.A, a.a_bytes);
+        const int q = lane % 8;
+#pragma unroll 1
+        for (int r = 8 * wave + lane / 8; r < BM; r += 8 * NW) {
             int any = 0;
-            for (int n = lane; n < cols; n += 64) any |= fabsf(ct[r * CS + n]) < doubt;
+            for (int n = q; n < cols; n += 8) any |= r < rows && fabsf(ct[r * CS + n]) < doubt;
             if (!__any(any)) continue;
-            const float *const row = a.A + (size_t)(m0 + r) * a.K;
             SbfRange x;
-#pragma unroll 8
-            for (int k = kbase + lane; k < kend; k += 64) x.see(row[k]);
+#pragma unroll 1
+            for (int kb = kbase; kb < kend; kb += 32 * 8) {
+                uintx4 w[8];
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
+                for (int u = 0; u < 8; ++u)
+                    w[u] = __builtin_amdgcn_raw_buffer_load_b128(
+                        rsa, ((unsigned)(m0 + r) * (unsigned)a.K + (unsigned)(kb + 32 * u + 4 * q)) * 4u, 0, 0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        x.see(kb + 32 * u + 4 * q + e < kend ? __uint_as_float(w[u][e]) : 0.0f);
+            }
+#pragma unroll
+            for (int o = 4; o > 0; o >>= 1) {
                 SbfRange y;
                 y.lo = (uint32_t)__shfl_xor((int)x.lo, o);
                 y.hi = (uint32_t)__shfl_xor((int)x.hi, o);
                 x.see(y);
             }
-            if (lane == 0) rrow[r] = x;
+            if (q == 0) rrow[r] = x;
         }
         __syncthreads();
         small = 0;
@@ -228,7 +306,7 @@ __device__ __forceinline__ void sbf_repair(const SbfArgs &a, float *ct, float *e
             if (grp < G) {
                 SbfRange x;
                 if (n < cols) {
-#pragma unroll 8
+#pragma unroll 16
                     for (int k = kbase + grp; k < kend; k += G) x.see(sbf_b<FMT>(a, k, n0 + n));
                 }
                 rcol[tid] = x;
@@ -253,11 +331,12 @@ __device__ __forceinline__ void sbf_repair(const SbfArgs &a, float *ct, float *e
         }
     }
 #pragma unroll 1
-    for (int e = tid; e < BM * BN; e += NT) {
-        const int r = e / BN, c = e % BN;
-        float *const v = &ct[r * CS + c];
-        if (r < rows && c < cols && sbf_not_finite(*v)) *v = sbf_fp32_sum<FMT>(a, m0 + r, n0 + c, kbase, kend);
-    }
+    for (int rb = 0; rb < BM / 32; ++rb)  // (blocks of a row, or of a column, on different waves)
+#pragma unroll 1
+        for (int cb = 0; cb < BN / 16; ++cb)
+            if ((rb + cb) % NW == wave)
+                sbf_recompute<FMT, CS, U>(a, ct + 32 * rb * CS + 16 * cb, m0 + 32 * rb, n0 + 16 * cb, rows - 32 * rb,
+                                       cols - 16 * cb, kbase, kend);
     __syncthreads();
 }
 
@@ -340,8 +419,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // against B's zero rows; B columns past N read the next k-row and feed dropped
     // outputs.  (A value there that is not finite makes its sum a NaN, which the
     // epilogue recomputes.)
-    constexpr unsigned ESZ = FMT == TML_FMT_F32 ? 4u : FMT == TML_FMT_F16 ? 2u : 1u;
-    auto col_bytes = [](unsigned n) constexpr { return kSbfStored<FMT> == TML_FMT_Q4_0 ? n / 2u : n * ESZ; };
+    auto col_bytes = [](unsigned n) constexpr { return kSbfStored<FMT> == TML_FMT_Q4_0 ? n / 2u : n * kSbfBytes<FMT>; };
     const unsigned b_bytes = (unsigned)kend * (unsigned)a.ldb;
     // A: AL loads 8 rows of 128 bytes an instruction (lane / 8, lane % 8), else 16
     // rows' 16-byte pieces in the MFMA's layout (c, g)
@@ -705,7 +783,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         if (kg == 0) put(true);
     }
     const bool suspect = worst >= 0x7F800000u - least_u || (TOP && top > 0x1p28f / kk);
-    if (__syncthreads_or(suspect))
+    if (__builtin_expect(__syncthreads_or(suspect), 0))
         sbf_repair<FMT, BM, BN, NW>(a, ct, ct + BM * CS, top, m0, n0, kbase, kend);
     constexpr int CH = BN / 4, RPP = NT / CH;  // 16-byte pieces of a tile row; rows a pass
     const int pc = 4 * (tid % CH), tr0 = tid / CH, col = n0 + pc;  // a thread's pieces lie in one column of pieces
