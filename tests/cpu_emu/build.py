@@ -31,7 +31,8 @@ FLAGS = ["-std=c++17", "-fno-omit-frame-pointer", "-fsanitize=address,undefined"
          "-I", HERE, "-I", CSRC, "-I", os.path.join(ROOT, "include"),
          # forced planner overrides at every size (the shipped library refuses
          # them above the sizes its GPU tests run them at)
-         "-DTML_FORCED_PLAN_MAX_MNK=0xFFFFFFFFFFFFFFFFull"]
+         # (EMU_FORCED_MAX of a case puts a limit back)
+         "-DTML_FORCED_PLAN_MAX_MNK=tml_emu_forced_max()"]
 
 sys.path.insert(0, ROOT)
 

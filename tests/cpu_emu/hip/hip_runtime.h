@@ -96,6 +96,11 @@ inline std::map<uintptr_t, size_t> &tml_emu_allocs() {
 // Non-zero makes hipStreamIsCapturing report an active capture.
 inline int tml_emu_capturing = 0;
 inline long long tml_emu_launches = 0;
+// The size above which the library refuses forced plans: none, or EMU_FORCED_MAX.
+inline uint64_t tml_emu_forced_max() {
+    const char *v = std::getenv("EMU_FORCED_MAX");
+    return v != nullptr ? std::strtoull(v, nullptr, 0) : ~0ull;
+}
 
 inline const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "emulated HIP error"; }
 inline hipError_t hipGetLastError() { return hipSuccess; }

@@ -378,3 +378,15 @@ def test_sbf_second_look(emu):
                     cases.append(f"gemm {fmt} 140 {n} {k} {flags} TML_GEMM_SBF_TILE={tile} TML_GEMM_SBF_SPLIT={split}")
     outs, fails = run_cases(emu, cases)
     assert not fails and not _err_lines(outs), (fails, _err_lines(outs)[:3])
+
+
+def test_forced_plans_refused_above_the_limit(emu):
+    # every override that forces a tile or a K split, just past a limit of 64 x 64 x 64 and at it
+    for key in ("TML_GEMM_TILE", "TML_GEMM_DMA_TILE", "TML_GEMM_SPLIT", "TML_GEMM_QBF_TILE", "TML_GEMM_QBF_SPLIT",
+                "TML_GEMM_SBF_TILE", "TML_GEMM_SBF_SPLIT"):
+        outs, fails = run_cases(emu, [f"gemm 0 {m} 64 64 b {key}=2 EMU_FORCED_MAX=262144" for m in (64, 65)], workers=1)
+        assert not fails and len(_ok_lines(outs)) == 1 and len(_err_lines(outs)) == 1, (key, outs)
+        assert "forced GEMM plans" in _err_lines(outs)[0] and "gemm 0 65" in _err_lines(outs)[0], (key, outs)
+    # a forced split is at most the planner's own: eight, unclamped, would not fit the static scratch
+    outs, fails = run_cases(emu, ["noalloc 0 512 1024 4096 - TML_GEMM_SBF_TILE=3 TML_GEMM_SBF_SPLIT=8"], workers=1)
+    assert not fails and len(_ok_lines(outs)) == 1, outs

@@ -979,6 +979,7 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 // call keeps being served under stream capture and without allocation.
 bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p) {
     constexpr double kCus = 256.0;
+    constexpr int kMaxSplit = 4;
     const bool is_int = sbf_fast(m), exact = sbf_int(m.fmt) && !is_int;
     const double mn = (double)m.M * (double)m.N;
     double best = other_us * (m.fmt == TML_FMT_F32 || is_int ? 1.1 : m.fmt == TML_FMT_Q8_K ? 0.95 : 1.0);
@@ -989,7 +990,7 @@ bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p
         if (rel == 0.0) continue;
         const int64_t tiles = ((m.M + t.bm - 1) / t.bm) * ((m.N + t.bn - 1) / t.bn);
         const int64_t slices = (m.K + t.bk - 1) / t.bk;
-        for (int s = 1; s <= 4; ++s) {
+        for (int s = 1; s <= kMaxSplit; ++s) {
             if (s > 1 && (tiles * s > 256 || slices / s < 8 || !m.sbf_split)) break;
             if (s > 1 && (is_int ? s > other_split : (double)s * mn > (double)kNoallocPartialFloats)) break;
             const double w = (double)(tiles * s) / kCus;  // tiles a CU
@@ -1018,7 +1019,7 @@ bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p
     const int forced = env_int("TML_GEMM_SBF_TILE", 0) - 1;
     if (sbf_cfg_ok(m, forced)) {
         cfg = forced;
-        nsplit = std::max(1, env_int("TML_GEMM_SBF_SPLIT", 1));
+        nsplit = m.sbf_split ? std::min(std::max(env_int("TML_GEMM_SBF_SPLIT", 1), 1), kMaxSplit) : 1;
     }
     if (cfg < 0) return false;
     const int64_t bk = kSbfCfgs[cfg].bk, slices = (m.K + bk - 1) / bk;
