@@ -20,7 +20,7 @@
 //          S allocates B 16 bytes short of its size (a planted mistake: the
 //          harness must report it); N makes the bf16 matrix cores return NaN
 //   NAME=VALUE  environment for this case only (the library's tuning overrides)
-// Output: "ok <line>" or "err <code> <message> <line>" per case; exit 0.
+// Output: "ok <launches> <line> wave_barriers=<of all threads>" or "err <code> <message> <line>" per case; exit 0.
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -195,12 +195,13 @@ int main() {
         }
         std::fprintf(stdout, "run %s\n", line.c_str());
         std::fflush(stdout);
-        const long long launches0 = tml_emu_launches;
+        const long long launches0 = tml_emu_launches, waves0 = tml_emu_wave_barriers;
         tml_emu_mfma_nan = op != "tlfile" && flags.find('N') != std::string::npos;
         const int rc = run_case(op, fmt, M, N, K, flags);
         for (auto &kv : env) unsetenv(kv.substr(0, kv.find('=')).c_str());
         if (rc == 0)
-            std::fprintf(stdout, "ok %lld %s\n", tml_emu_launches - launches0, line.c_str());
+            std::fprintf(stdout, "ok %lld %s wave_barriers=%lld\n", tml_emu_launches - launches0, line.c_str(),
+                         tml_emu_wave_barriers - waves0);
         else
             std::fprintf(stdout, "err %d [%s] %s\n", rc, tml_hip_last_error(), line.c_str());
         std::fflush(stdout);

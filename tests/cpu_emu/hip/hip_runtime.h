@@ -284,7 +284,8 @@ inline void __builtin_amdgcn_s_waitcnt(int) {}
 inline void __builtin_amdgcn_s_barrier() {}
 inline void __builtin_amdgcn_sched_barrier(int) {}
 inline void __builtin_amdgcn_sched_group_barrier(int, int, int) {}
-inline void __builtin_amdgcn_wave_barrier() {}
+inline long long tml_emu_wave_barriers = 0;
+inline void __builtin_amdgcn_wave_barrier() { ++tml_emu_wave_barriers; }
 inline void __builtin_amdgcn_fence(int, const char *) {}
 template <typename T>
 inline T __builtin_amdgcn_readfirstlane(T v) {

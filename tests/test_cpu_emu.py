@@ -390,3 +390,15 @@ def test_forced_plans_refused_above_the_limit(emu):
     # a forced split is at most the planner's own: eight, unclamped, would not fit the static scratch
     outs, fails = run_cases(emu, ["noalloc 0 512 1024 4096 - TML_GEMM_SBF_TILE=3 TML_GEMM_SBF_SPLIT=8"], workers=1)
     assert not fails and len(_ok_lines(outs)) == 1, outs
+
+
+def test_sbf_int_wave_exchange(emu):
+    # int8 / int4 turn A through LDS rows of one wave: a wave barrier between the lanes'
+    # writes and their reads, and one before the next writes, for each 16-row tile (two a wave)
+    # of each 32-deep slice
+    for tile, tiles in ((1, 1), (2, 2)):
+        for fmt in (Q8_0, Q4_0):
+            outs, fails = run_cases(emu, [f"gemm {fmt} 40 128 96 b TML_GEMM_SBF_TILE={tile}"], workers=1)
+            assert not fails and len(_ok_lines(outs)) == 1, outs
+            n = int(_ok_lines(outs)[0].rsplit("=", 1)[1])
+            assert n >= tiles * 512 * 3 * 2 * 2, (tile, fmt, n)

@@ -477,8 +477,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         }
     };
 
-    // AL: rows 16 i + 8 h .. + 7 through the wave's own LDS rows (no barrier: one
-    // wave's LDS accesses run in order), 16-byte chunk q of row r in slot q ^ (r % 8).
+    // AL: rows 16 i + 8 h .. + 7 through the wave's own LDS rows (no workgroup barrier: one
+    // wave's LDS accesses run in order, and turn() keeps the compiler's order of the
+    // lanes' writes and reads), 16-byte chunk q of row r in slot q ^ (r % 8).
+    auto turn = []() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
     uintx4 *const aw = lds + kARows + wave * (WM * 8);
     const int slot_aw = lane / 8 * 8 + (lane % 8 ^ lane / 8), slot_ar = c * 8 + (g ^ (c & 7));
     uint32_t rr[TM][8];
@@ -628,6 +634,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
                         if (write_a_at(i) == gi) {
+                            turn();
 #pragma unroll
                             for (int h = 0; h < 2; ++h) {
                                 write_a(i, h, da);
@@ -636,7 +643,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
                         }
 #pragma unroll
                     for (int i = 0; i < TM; ++i)
-                        if (read_a_at(i) == gi) read_a(i);
+                        if (read_a_at(i) == gi) {
+                            turn();
+                            read_a(i);
+                        }
                 }
 #pragma unroll
                 for (int v = 0; v < kSplits; ++v)
@@ -712,6 +722,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         for (int i = 0; i < TM; ++i) {
             write_a(i, 0, 0);
             write_a(i, 1, 0);
+            turn();
             read_a(i);
         }
     }
