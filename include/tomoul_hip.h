@@ -149,7 +149,7 @@ int tml_hip_sgemm_q8(int64_t M, int64_t N, int64_t K, const float *A, const int8
  * entry point): fp32 multiply-adds on the fp32 matrix cores, or -- where that is
  * faster, the larger products -- the bf16 matrix cores with every operand split
  * exactly into bf16 terms and the products of the terms summed in fp32, dropped
- * terms below 2^-25 of a product; both are fp32 results (2-norm error against 64
+ * terms at most 2^-24 of a product (F16 weights: 2^-25); both are fp32 results (2-norm error against 64
  * bits 1e-7 to 1e-6).  Outputs that the terms cannot carry -- infinities, NaNs,
  * operands past the largest bf16, sums (zero included) that an operand below 2^-102
  * or a product below 2^-80 may have put off by 2^-24 of themselves -- are

@@ -3,7 +3,7 @@
 Every operand is split exactly into bf16 terms and the products of the terms
 that matter are summed in fp32, so an output differs from the 64-bit product
 of the same operands by at most one fp32 rounding of each 32-deep slice's sum,
-the six dropped or merged small terms (below 2^-24 of a product together) and
+the small terms, dropped (at most 2^-24 of a product together) or summed apart, and
 the epilogue's own roundings:
     |C - ref| <= (ceil(K / 32) + 8) * 2^-24 * sum_k |a b| + 2^-23 |ref|.
 Outputs the split does not carry (infinities, NaNs, values past the largest

@@ -7,14 +7,14 @@
 // The reference's products are fp32 (src/core/ops.zig:277-414; f16 and Q8_K
 // weights widened to f32, src/core/quantization.zig:559-614, :1921-1962).  An
 // fp32 value's 24 bits are three bf16 terms, x = h + m + l, each the nearest
-// bf16 of what the ones before leave (|m| <= 2^-9 |x|, |l| <= 2^-18 |x|, the
+// bf16 of what the ones before leave (|m| <= 2^-8 |x|, |l| <= 2^-17 |x|, the
 // sum exact), so
-//   a . b = hh + hm + mh + mm + hl + lh  (+ ml + lm + ll, at most 2^-25 |a b|)
+//   a . b = hh + hm + mh + mm + hl + lh  (+ ml + lm + ll, at most 2^-24 |a b|)
 // with every kept product exact.  Six v_mfma_f32_16x16x32_bf16 (five for f16
 // weights, whose 11 bits are two bf16 terms, h + m, exactly) do the work of eight
 // v_mfma_f32_16x16x4_f32 at 16 times their rate: 2.5 PFLOP/s / 6 = 417 against 157
-// TFLOP/s.  The dropped terms are below half an fp32 rounding of the product, and
-// the hh products have an accumulator of their own, which a 32-deep slice rounds
+// TFLOP/s.  The dropped terms (for f16 weights lm alone, 2^-25) are at most one fp32
+// rounding of the product, and the hh products have an accumulator of their own, which a 32-deep slice rounds
 // once where the fp32 matrix cores round theirs eight times: the 2-norm error
 // against 64 bits is 0.9e-7 - 4.5e-7 over the shapes at pick_sbf, theirs 3.7e-7 -
 // 9.9e-7.
