@@ -903,9 +903,13 @@ bool sbf_int(int fmt) { return fmt == TML_FMT_Q8_0 || fmt == TML_FMT_Q4_0; }
 // boundary), where the fp32 matrix cores' general kernel ran: at its precision.
 bool sbf_exact(const MatmulArgs &m) { return sbf_int(m.fmt) && !gemm_qbf_supported(m); }
 bool sbf_fast(const MatmulArgs &m) { return sbf_int(m.fmt) && gemm_qbf_supported(m); }
+// A slice's cost in m's format, relative to f32; 0 where the tile has no kernel for it.
+double sbf_cost(const MatmulArgs &m, const SbfCfg &t) {
+    return m.fmt == TML_FMT_F16 ? t.f16 : m.fmt == TML_FMT_Q8_K ? t.q8k : sbf_exact(m) ? t.exact : 1.0;
+}
 bool sbf_cfg_ok(const MatmulArgs &m, int c) {
     if (sbf_fast(m)) return c >= 0 && c < kSbfNumIntCfgs;
-    return c >= 0 && c < kSbfNumCfgs && (!sbf_int(m.fmt) || kSbfCfgs[c].exact > 0.0);
+    return c >= 0 && c < kSbfNumCfgs && sbf_cost(m, kSbfCfgs[c]) > 0.0;
 }
 
 template <int FMT>
@@ -922,7 +926,10 @@ void launch_sbf_cfg(int cfg, unsigned grid, const SbfArgs &a, hipStream_t s) {
         }
     } else {
         switch (cfg) {  // (the large tiles' registers hold one slice of loads ahead)
-            case 0: gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
+            case 0:  // (Q8_K: more registers than there are)
+                if constexpr (FMT != TML_FMT_Q8_K)
+                    gemm_sbf_kernel<FMT, 256, 128, 32, 128, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a);
+                break;
             case 1: gemm_sbf_kernel<FMT, 256, 96, 32, 96, 32, 1, 8, 1><<<grid, 512, 0, s>>>(a); break;
             case 2: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 64, 2, 8, 2><<<grid, 512, 0, s>>>(a); break;
             case 3: gemm_sbf_kernel<FMT, 128, 64, 32, 64, 32, 1, 4, 2><<<grid, 256, 0, s>>>(a); break;
@@ -991,13 +998,13 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 bool pick_sbf(const MatmulArgs &m, double other_us, int other_split, GemmPlan *p) {
     constexpr double kCus = 256.0;
     constexpr int kMaxSplit = 4;
-    const bool is_int = sbf_fast(m), exact = sbf_int(m.fmt) && !is_int;
+    const bool is_int = sbf_fast(m);
     const double mn = (double)m.M * (double)m.N;
     double best = other_us * (m.fmt == TML_FMT_F32 || is_int ? 1.1 : m.fmt == TML_FMT_Q8_K ? 0.95 : 1.0);
     int cfg = -1, nsplit = 1;
     for (int c = 0; c < (is_int ? kSbfNumIntCfgs : kSbfNumCfgs); ++c) {
         const SbfCfg &t = is_int ? kSbfIntCfgs[c] : kSbfCfgs[c];
-        const double rel = m.fmt == TML_FMT_F16 ? t.f16 : m.fmt == TML_FMT_Q8_K ? t.q8k : exact ? t.exact : 1.0;
+        const double rel = is_int ? 1.0 : sbf_cost(m, t);
         if (rel == 0.0) continue;
         const int64_t tiles = ((m.M + t.bm - 1) / t.bm) * ((m.N + t.bn - 1) / t.bn);
         const int64_t slices = (m.K + t.bk - 1) / t.bk;

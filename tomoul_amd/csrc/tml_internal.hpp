@@ -219,8 +219,8 @@ double pick_qbf(const MatmulArgs &a, GemmPlan *p);
 Status launch_gemm_qbf(const MatmulArgs &a, const GemmPlan &p, const Workspace &ws, hipStream_t s);
 // GEMM on the bf16 matrix cores with the operands split into bf16 terms
 // (gemm_sbf.hip): M > kGemvMaxM, any K and N (int4: even N; Q8_K: N % 32 == 0 and blocks
-// of 32), A on a 4-byte boundary, B on its element's.  pick_sbf is false where the other kernels, at a modelled other_us with other_split K splits, are
-// the faster choice.
+// of 32), A on a 4-byte boundary, B on its element's.  pick_sbf is false where the
+// other kernels, at a modelled other_us with other_split K splits, are the faster choice.
 bool gemm_sbf_supported(const MatmulArgs &a);
 bool pick_sbf(const MatmulArgs &a, double other_us, int other_split, GemmPlan *p);
 Status launch_gemm_sbf(const MatmulArgs &a, const GemmPlan &p, const Workspace &ws, hipStream_t s);
