@@ -134,8 +134,8 @@ int tml_hip_sgemm_q8(int64_t M, int64_t N, int64_t K, const float *A, const int8
  * GEMV takes, they run on the bf16 matrix cores, the int weights exact in
  * bf16 and each fp32 activation split into two bf16 terms
  * (|x - hi - lo| <= 2^-17 |x|), accumulated in fp32; outside those layouts
- * (M > 8, and K % 4 != 0, N % 8 != 0 or an operand whose alignment leaves no wide
- * loads) with an exact three-term split; otherwise on fp32 multiply-adds.  All agree with
+ * (M > 8) with an exact three-term split, or, where K % 4 == 0, N % 8 == 0 and the
+ * product is small, as everywhere else, on fp32 multiply-adds.  All agree with
  * the reference's dequantize-then-fp32-accumulate result to ~1e-5 relative;
  * infinities and NaNs in A give what the reference gives.  Limit: the
  * per-tensor scale multiplies the finished sum (the reference multiplies

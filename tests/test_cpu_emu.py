@@ -402,3 +402,18 @@ def test_sbf_int_wave_exchange(emu):
             assert not fails and len(_ok_lines(outs)) == 1, outs
             n = int(_ok_lines(outs)[0].rsplit("=", 1)[1])
             assert n >= tiles * 512 * 3 * 2 * 2, (tile, fmt, n)
+
+
+def test_sbf_int_rule(emu):
+    # int8 / int4 outside the bf16 kernel's layouts reach the split-bf16 kernel at every K
+    # that is no multiple of 8 (shown by a K split that only it has at this depth)
+    for fmt in (Q8_0, Q4_0, Q8_0_PC):
+        for k in (97, 98, 100, 102, 103, 108):
+            outs, fails = run_cases(emu, [f"gemm {fmt} 70 64 {k} b TML_GEMM_SBF_TILE=5 TML_GEMM_SBF_SPLIT=2 "
+                                          "TML_REQUIRE_SPLIT=1"], workers=1)
+            assert not fails and len(_ok_lines(outs)) == 1, (fmt, k, outs)
+    # the default plan at sizes on both sides of the model, wide loads or not
+    cases = [f"gemm {fmt} {m} {n} {k} br" for fmt in (Q8_0, Q4_0) for (m, n, k) in
+             [(300, 1344, 516), (20, 328, 500), (257, 1000, 132), (1500, 1536, 100), (40, 98, 388)]]
+    outs, fails = run_cases(emu, cases)
+    assert not fails and not _err_lines(outs), (fails, _err_lines(outs)[:3])

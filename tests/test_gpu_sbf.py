@@ -263,6 +263,20 @@ def test_sbf_int_exact(orc, env, tile, split):
                   orc.dequantize_q4(p, k * n, s4).reshape(k, n), bias.astype(np.float64))
 
 
+@pytest.mark.parametrize("fmt", [_abi.FMT_Q8_0, _abi.FMT_Q4_0])
+@pytest.mark.parametrize("m,n,k", [(1500, 1536, 388), (600, 1000, 1028), (20, 1000, 132)])
+def test_sbf_int_k4(orc, fmt, m, n, k):
+    # K % 8 == 4 with wide loads, the planner's own choice: the split-bf16 kernel at the
+    # largest, the fp32-MFMA kernels (600 x 1000 has few tiles) at the others
+    a, bias, w = synth.normal_matrix(121, m, k), synth.normal(122, n, 0.0, 0.02), synth.normal_matrix(123, k, n, 0.02)
+    q, s = (orc.quantize_q8 if fmt == _abi.FMT_Q8_0 else orc.quantize_q4)(w)
+    deq = (orc.dequantize_q8(q, s) if fmt == _abi.FMT_Q8_0 else orc.dequantize_q4(q, k * n, s)).reshape(k, n)
+    c = run(fmt, m, n, k, a, q, None, scale=s, bias=bias)
+    ref = a.astype(np.float64) @ deq.astype(np.float64) + bias
+    # 2-norm: 0.6e-7 - 2.8e-7 on the split kernel, up to 9.9e-7 on the fp32 matrix cores
+    assert np.linalg.norm(c - ref) <= (3e-7 if m == 1500 else 1e-6) * np.linalg.norm(ref)
+
+
 @pytest.mark.parametrize("tile", [1, 2])
 def test_sbf_int_inf_nan(orc, env, tile):
     env["TML_GEMM_SBF_TILE"] = str(tile)

@@ -687,15 +687,17 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
         few_tiles = tiles < cus / 2 || (tiles < cus && m.K >= 2048);
     }
     double other_us = 1e300;  // modelled time of the fp32-MFMA plan
+    const bool is_int = m.fmt == TML_FMT_Q8_0 || m.fmt == TML_FMT_Q4_0;
+    const bool int_wide = m.K % 4 == 0 && m.N % 8 == 0 && aligned(m.A, 16) && aligned(m.B, m.fmt == TML_FMT_Q4_0 ? 4 : 8);
     const bool by_m = m.fmt == TML_FMT_F16 || (m.fmt == TML_FMT_Q8_K && !(m.M >= 512 && m.N >= 4096)) ||
                       (m.fmt == TML_FMT_Q4_0 && (m.M >= 1024 || m.M <= 128));
     const bool narrow_ok = m.fmt == TML_FMT_F32 || dma_q == 1 || (dma_q < 0 && (by_m || few_tiles));
     if (narrow_ok && env_int("TML_GEMM_DMA", 1) != 0 && gemm_dma_supported(m) && m.K > 0) {
         p.dma = true;
         other_us = pick_dma(m.M, m.N, m.K, m.fmt, &p);
-    } else if (gemm_dma_supported(m) && m.K > 0) {
+    } else if ((is_int ? int_wide : gemm_dma_supported(m)) && m.K > 0) {
         // the register-staged kernel, within a few per cent of the direct-copy
-        // one where it is preferred
+        // one where it is preferred (int8 / int4 of N % 8 == 0: its own wide loads)
         GemmPlan unused;
         other_us = pick_dma(m.M, m.N, m.K, m.fmt, &unused);
     }
@@ -704,12 +706,16 @@ GemmPlan plan_gemm(const MatmulArgs &m) {
     // asks for one of the fp32-MFMA kernels.
     const bool other_forced = fp32_forced || set("TML_GEMM_DMA") || set("TML_GEMM_FUSED") || set("TML_GEMM_XCDPART") ||
                               set("TML_GEMM_XCD") || set("TML_GEMM_GROUPM");
-    // Int8 / int4 outside gemm_qbf.hip's layouts likewise, where the register-staged
-    // kernel would read them element by element (its own override, TML_GEMM_QBF, aside).
+    // Int8 / int4 likewise: here they are outside gemm_qbf.hip's layouts (or that
+    // kernel's own override, TML_GEMM_QBF, turns it off).  Where rows are whole wide loads
+    // (int_wide: K % 8 == 4 here) the fp32-MFMA kernels' plan is modelled and stays where few
+    // tiles favour it; us, those kernels / the split-bf16 one: Q8_0 1500x3840x1284 132 / 56.6,
+    // 1500x1536x388 29.2 / 18.5, 512x4096x1028 45.6 / 25.5, 2500x3008x2004 260 / 138 (Q4_0
+    // 142 / 53.8, 26.5 / 17.1, 42.9 / 24.4, 282 / 136); unpicked: 278x1344x2236 29.7, 300x1000x1028
+    // 17.5, 60x512x396 7.0.
+    // Elsewhere they would be read element by element, and no model stands against it.
     GemmPlan q;
-    const bool is_int = m.fmt == TML_FMT_Q8_0 || m.fmt == TML_FMT_Q4_0;
-    const bool int_ok = m.K % 4 != 0 || m.N % 8 != 0 || !aligned(m.A, 16) || !aligned(m.B, m.fmt == TML_FMT_Q4_0 ? 4 : 8);
-    if (!other_forced && (!is_int || (int_ok && !set("TML_GEMM_QBF"))) && gemm_sbf_supported(m) &&
+    if (!other_forced && (!is_int || !set("TML_GEMM_QBF")) && gemm_sbf_supported(m) &&
         pick_sbf(m, other_us, p.nsplit, &q)) {
         q.sbf = true;
         return q;
