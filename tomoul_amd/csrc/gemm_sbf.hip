@@ -381,7 +381,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     constexpr int CS = BN + 4;            // floats of a staged C row (rows 4 apart: 16 banks on)
     constexpr int kARows = 3 * kStage;    // AL: the waves' own A rows, WM x 8 slots each
     constexpr int kLoop = kARows + (AL ? NW * WM * 8 : 0);
-    constexpr int kTile = (BM * CS + kSbfRepairFloats<BM, BN, NW>) / 4;  // the epilogue's
+    constexpr int kTile = (BM * CS + kSbfRepairFloats<BM, BN, NW> + NW) / 4;  // the epilogue's
     constexpr int kLds = kLoop > kTile ? kLoop : kTile;
     __shared__ uintx4 lds[kLds];
 
@@ -763,13 +763,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // activation in every element it cost 36 k cycles a tile (16 of the 102 us of
     // 1500x5120x1280).
     float *const ct = (float *)lds;
-    // not finite, or below `least` (no less than sbf_doubt, top permitting); of the
-    // rows and columns past the matrix, whose sums are zeros, none is looked at
+    // not finite, or below `least` (no less than sbf_doubt, top permitting).  Rows past M,
+    // whose sums are zeros, are not looked at; columns past N hold other columns' products
     const float kk = (float)(kend - kbase), least = fmaxf(0x1p-70f, sbf_doubt(kk, kSbfTopB<FMT>));
-    const uint32_t least_u = __float_as_uint(least);
+    const uint32_t least2 = __float_as_uint(least) << 1;  // (the sign shifted out)
     uint32_t worst = 0;
     auto put = [&](bool add) __attribute__((always_inline)) {
-        const int rows = a.M - m0 - wm0 - 4 * g, cols = a.N - n0 - wn0 - c;
+        const int rows = a.M - m0 - wm0 - 4 * g;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -779,7 +779,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
                 for (int j = 0; j < TN; ++j) {
                     float *const to = &ct[(wm0 + 16 * i + 4 * g + e) * CS + wn0 + 16 * j + c];
                     const float v = add ? *to + acc[i][j][e] : acc[i][j][e];
-                    w = max(w, 16 * j < cols ? (__float_as_uint(v) & 0x7FFFFFFFu) - least_u : 0u);
+                    w = max(w, (__float_as_uint(v) << 1) - least2);
                     *to = v;
                 }
                 worst = max(worst, 16 * i + e < rows ? w : 0u);
@@ -793,8 +793,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         __syncthreads();
         if (kg == 0) put(true);
     }
-    const bool suspect = worst >= 0x7F800000u - least_u || (TOP && top > 0x1p28f / kk);
-    if (__builtin_expect(__syncthreads_or(suspect), 0))
+    const bool suspect = worst >= 0xFF000000u - least2 || (TOP && top > 0x1p28f / kk);
+    // (each wave's flag in LDS past sbf_repair's floats: one barrier, where __syncthreads_or has two)
+    uint32_t *const flags = (uint32_t *)(ct + BM * CS + kSbfRepairFloats<BM, BN, NW>);
+    const bool mine = __any(suspect);
+    if (lane == 0) flags[wave] = mine;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) any |= flags[w];
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(any) != 0, 0))
         sbf_repair<FMT, BM, BN, NW>(a, ct, ct + BM * CS, top, m0, n0, kbase, kend);
     constexpr int CH = BN / 4, RPP = NT / CH;  // 16-byte pieces of a tile row; rows a pass
     const int pc = 4 * (tid % CH), tr0 = tid / CH, col = n0 + pc;  // a thread's pieces lie in one column of pieces
