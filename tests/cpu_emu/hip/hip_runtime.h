@@ -240,6 +240,7 @@ tml_emu_launcher<P...> tml_emu_launch(void (*k)(P...), dim3 g, dim3 b, size_t sh
 inline void __syncthreads() {}
 inline int __syncthreads_or(int v) { return v; }
 inline int __any(int v) { return v; }
+inline uint64_t __builtin_amdgcn_ballot_w64(bool v) { return v ? ~0ull : 0ull; }
 template <typename A, typename B>
 inline std::common_type_t<A, B> min(A a, B b) {
     return a < b ? a : b;

@@ -199,6 +199,29 @@ def test_sbf_small_operands_formats(orc, env, tile, fmt, ea, ew):
     assert np.all(np.abs(c - ref) <= k * 2.0**-24 * mag), float(np.max(np.abs(c - ref) / mag))
 
 
+@pytest.mark.parametrize("tile,split", [(t, 1) for t in TILES] + [(3, 2), (5, 3)])
+@pytest.mark.parametrize("k", [128, 100])
+def test_sbf_zero_rows(env, tile, split, k):
+    # rows of zeros between others (k = 100: the last slice reads on into the next row):
+    # zeros, a NaN where the weight is infinite, and a zero where it is past the largest bf16;
+    # a row of zeros and one NaN
+    env["TML_GEMM_SBF_TILE"], env["TML_GEMM_SBF_SPLIT"] = str(tile), str(split)
+    m, n = 140, 101
+    a, w = synth.normal_matrix(131, m, k), synth.normal_matrix(132, k, n, 0.02)
+    zero = np.r_[2, 17:40, 63, 64, 100:140]
+    a[zero] = 0.0
+    a[17, 3] = np.nan
+    w[5, 9], w[k - 1, 50], w[:, 70] = np.inf, np.float32(3.4028235e38), 0.0
+    c = run(_abi.FMT_F32, m, n, k, a, w, None)
+    with np.errstate(invalid="ignore", over="ignore"):  # (column 50 overflows fp32 where |a| > 1)
+        ref = (a.astype(np.float64) @ w.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(np.isnan(c), np.isnan(ref)) and np.array_equal(np.isinf(c), np.isinf(ref))
+    rows = np.isfinite(a).all(1)
+    assert np.all(c[zero][rows[zero]][:, np.arange(n) != 9] == 0.0) and np.all(c[rows][:, 70] == 0.0)
+    cols = ~np.isin(np.arange(n), (9, 50))
+    check(c[rows][:, cols], a[rows], w[:, cols])
+
+
 def test_sbf_exact_integers(env):
     # products and sums of small integers are exact
     rng = np.random.default_rng(5)

@@ -37,9 +37,9 @@
 // the largest of the other operand, and by K 2^-122 where products of terms
 // themselves fall below 2^-126.  An output smaller than 2^24 times what it may be off by
 // -- zero included -- is recomputed from the operands (sbf_repair), as is one that
-// is not finite.  The split notes the largest magnitude that passes through it (one
-// v_max3 a pair of values, 11 instructions before), so outputs of 2^-70 and more need no second look
-// unless an operand is past 2^28 / K.
+// is not finite.  The split notes the largest magnitudes that pass through it (one
+// v_max3 a pair of values, 11 instructions before), so outputs of 2^-70 and more need no
+// second look unless an operand is past 2^28 / K, nor do those of a row of zeros.
 #include "tml_internal.hpp"
 
 #include <algorithm>
@@ -238,7 +238,8 @@ struct SbfRange {
 // Puts right the outputs in ct, the tile's sums over k in [kbase, kend), that the split
 // does not carry (top of the file).  Small ones are first weighed by what their own
 // row of A and column of B hold: a sum of zeros, or of values that cancel, is as good as
-// any, and rows of zeros are told apart before any column is read.  top: the
+// any, and rows of zeros are told apart before any column is read.  512x4096x1024 f32 with
+// one column of zeros: 50 us, 29 without (cold instructions, then the loads' latency).  top: the
 // largest magnitude this lane has split.  ex: LDS, sbf_repair_floats floats.
 template <int BM, int BN, int NW>
 constexpr int kSbfRepairFloats = 2 * (BM + 64 * NW);
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     constexpr int CS = BN + 4;            // floats of a staged C row (rows 4 apart: 16 banks on)
     constexpr int kARows = 3 * kStage;    // AL: the waves' own A rows, WM x 8 slots each
     constexpr int kLoop = kARows + (AL ? NW * WM * 8 : 0);
-    constexpr int kTile = (BM * CS + kSbfRepairFloats<BM, BN, NW> + NW) / 4;  // the epilogue's
+    constexpr int kTile = (BM * CS + kSbfRepairFloats<BM, BN, NW> + NW + (KW == 2 ? NWS * (WM / 16) : 0)) / 4;  // the epilogue's
     constexpr int kLds = kLoop > kTile ? kLoop : kTile;
     __shared__ uintx4 lds[kLds];
 
@@ -415,8 +416,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
 
     // ---- loads.  A lane's offsets are fixed; the slice moves the buffer's base
     // and byte count (scalar work only).  Rows of A past M and k-rows of B past
-    // kend lie past the byte count and read zeros.  A's k past kend reads on,
-    // against B's zero rows; B columns past N read the next k-row and feed dropped
+    // kend lie past the byte count and read zeros, as does a slice of A past kend.  A's k past
+    // kend in the last slice reads on, against B's zero rows; B columns past N read the next k-row and feed dropped
     // outputs.  (A value there that is not finite makes its sum a NaN, which the
     // epilogue recomputes.)
     auto col_bytes = [](unsigned n) constexpr { return kSbfStored<FMT> == TML_FMT_Q4_0 ? n / 2u : n * kSbfBytes<FMT>; };
@@ -441,7 +442,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     };
     // the buffers at a slice's first k
     auto at_a = [&](int k0) __attribute__((always_inline)) {
-        return moved(a.A, a.a_bytes, ((unsigned)(m0 + wm0) * (unsigned)a.K + (unsigned)(kbase + k0 + 32 * kg)) * 4u);
+        const int k = kbase + k0 + 32 * kg;
+        return moved(a.A, a.a_bytes, k < kend ? ((unsigned)(m0 + wm0) * (unsigned)a.K + (unsigned)k) * 4u : a.a_bytes);
     };
     auto at_b = [&](int k0) __attribute__((always_inline)) {
         return moved(a.B, b_bytes, (unsigned)(kbase + k0) * (unsigned)a.ldb + col_bytes((unsigned)n0));
@@ -504,9 +506,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // ---- splitting, a pair of k at a time: A's pair e to word e of the next
     // slice's operands, B's to word e of the slots write_b stores.
     constexpr bool TOP = kSbfTopB<FMT> == 0.0f;
-    float top = kSbfTopB<FMT>;  // the largest magnitude split
-    auto note = [&](float x, float y) __attribute__((always_inline)) {
-        if constexpr (TOP) top = fmaxf(fmaxf(top, fabsf(x)), fabsf(y));
+    // the largest magnitudes split: of B, and of A's row 16 i + c (with B bounded by its
+    // format, to tell rows of zeros; two terms of A do without)
+    float top_b = kSbfTopB<FMT>, top_a[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) top_a[i] = 0.0f;
+    auto note = [&](float &t, float x, float y) __attribute__((always_inline)) {
+        t = fmaxf(fmaxf(t, fabsf(x)), fabsf(y));
     };
     uintx4 av[2][NA][TM], bp[PB][NB];
     float bx[PB][4][2];  // B's values, for note()
@@ -514,7 +520,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         uint32_t t[NA];
         const float x = __uint_as_float(AL ? rr[i][2 * e] : ra[d][i][2 * e]);
         const float y = __uint_as_float(AL ? rr[i][2 * e + 1] : ra[d][i][2 * e + 1]);
-        note(x, y);
+        if constexpr (COR) note(top_a[i], x, y);
         sbf_split<NA>(x, y, t);
 #pragma unroll
         for (int p = 0; p < NA; ++p) av[nxt][p][i][e] = t[p];
@@ -539,9 +545,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     auto write_b = [&](int t, int p, int stage) __attribute__((always_inline)) {
         if (TB % NT == 0 || tid + t * NT < TB) {
             lds[stage + slot_b[t] + p * BN * SL] = bp[t][p];
-            if (p == 0) {  // (here, so that threads without a task split nothing: noted in split_b, 9-16 registers more)
+            if (TOP && p == 0) {  // (here, so that threads without a task split nothing: noted in split_b, 9-16 registers more)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) note(bx[t][e][0], bx[t][e][1]);
+                for (int e = 0; e < 4; ++e) note(top_b, bx[t][e][0], bx[t][e][1]);
             }
         }
     };
@@ -767,6 +773,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
     // whose sums are zeros, are not looked at; columns past N hold other columns' products
     const float kk = (float)(kend - kbase), least = fmaxf(0x1p-70f, sbf_doubt(kk, kSbfTopB<FMT>));
     const uint32_t least2 = __float_as_uint(least) << 1;  // (the sign shifted out)
+    uint32_t *const flags = (uint32_t *)(ct + BM * CS + kSbfRepairFloats<BM, BN, NW>);
+    // rows of zeros (their lanes c, c + 16, c + 32, c + 48 met nothing else), a bit each
+    uint32_t zeros[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const uint64_t z = COR ? __builtin_amdgcn_ballot_w64(top_a[i] == 0.0f) : 0;
+        zeros[i] = (uint32_t)(z & z >> 16 & z >> 32 & z >> 48) & 0xFFFFu;
+    }
     uint32_t worst = 0;
     auto put = [&](bool add) __attribute__((always_inline)) {
         const int rows = a.M - m0 - wm0 - 4 * g;
@@ -774,28 +788,43 @@ __global__ __launch_bounds__(64 * NW) void gemm_sbf_kernel(SbfArgs a) {
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                uint32_t w = 0;
+                uint32_t w = 0, any = 0;
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
                     float *const to = &ct[(wm0 + 16 * i + 4 * g + e) * CS + wn0 + 16 * j + c];
                     const float v = add ? *to + acc[i][j][e] : acc[i][j][e];
-                    w = max(w, (__float_as_uint(v) << 1) - least2);
+                    const uint32_t u = __float_as_uint(v) << 1;
+                    // (two terms of A: a zero sum is taken as it is, as in gemm_qbf.hip)
+                    w = max(w, (COR || u != 0 ? u : least2) - least2);
+                    any |= u;
                     *to = v;
                 }
+                if (COR && (zeros[i] >> (4 * g + e) & 1) && any == 0) w = 0;
                 worst = max(worst, 16 * i + e < rows ? w : 0u);
             }
     };
     if constexpr (KW == 1) {
         put(false);
     } else {
-        if (kg == 1) put(false);
+        if (kg == 1) {
+            put(false);
+#pragma unroll
+            for (int i = 0; i < TM && COR; ++i)
+                if (lane == 0) flags[NW + sw * TM + i] = zeros[i];
+        }
         worst = 0;
         __syncthreads();
-        if (kg == 0) put(true);
+        if (kg == 0) {
+#pragma unroll
+            for (int i = 0; i < TM && COR; ++i) zeros[i] &= flags[NW + sw * TM + i];
+            put(true);
+        }
     }
+    float top = top_b;
+#pragma unroll
+    for (int i = 0; i < TM && TOP; ++i) top = fmaxf(top, top_a[i]);
     const bool suspect = worst >= 0xFF000000u - least2 || (TOP && top > 0x1p28f / kk);
     // (each wave's flag in LDS past sbf_repair's floats: one barrier, where __syncthreads_or has two)
-    uint32_t *const flags = (uint32_t *)(ct + BM * CS + kSbfRepairFloats<BM, BN, NW>);
     const bool mine = __any(suspect);
     if (lane == 0) flags[wave] = mine;
     __syncthreads();
