@@ -23,17 +23,19 @@
 // layouts, where the fp32 matrix cores' general kernel ran, A takes three terms and
 // the products are three: fp32 precision as before.
 //
-// Bound: the matrix cores, at the clock the power limit leaves them.  At
-// 1500x5120x1280 (240 tiles of 256x128) the main loop keeps them 82 % busy, at
-// 1.85 GHz (2.3 GHz with 48 CUs busy): 95 us, 207 TFLOP/s, 165 us before on the
-// fp32 matrix cores.  Int8, same shape: 49 us, 401 TFLOP/s of algorithmic work; its
-// two products take a third of the matrix-core time, and LDS and the loads' issue
-// are as large.
+// Bound: issue beside the matrix cores -- two (256x128) to three and a half (128x64) other
+// vector instructions an MFMA, most of them the split's -- then fill and epilogue, at the clock the power limit
+// leaves (1.94 GHz with 240 CUs busy, 2.3 with 48).  The counters have the matrix cores
+// busy 69 % of a launch's CU cycles at 1500x5120x1280 (240 tiles of 256x128: 92 us, 214
+// TFLOP/s, 162 us before on the fp32 matrix cores), 63 % on 256x96 tiles at
+// 1500x3840x1280 (75 us) and 54 % on 128x64 tiles at 1500x1280x5120 (115 us).  Int8,
+// 1500x5120x1280: 46 us, 427 TFLOP/s of algorithmic work; its two products take a third of
+// the matrix-core time, and LDS and the loads' issue are as large.
 //
 // Values the split does not carry.  Infinities, NaNs (their residual is NaN) and
 // |x| above the largest bf16 make the sum infinite or NaN.  Of a nonzero |x| < 2^-102
-// up to 2^-124 may be lost (its terms reach bf16's denormals; the largest value
-// below 2^-134 has none at all), so a sum of K products is off by up to K 2^-124 times
+// up to 2^-124 may be lost (its terms reach bf16's denormals; values
+// below 2^-134 have none at all), so a sum of K products is off by up to K 2^-124 times
 // the largest of the other operand, and by K 2^-122 where products of terms
 // themselves fall below 2^-126.  An output smaller than 2^24 times what it may be off by
 // -- zero included -- is recomputed from the operands (sbf_repair), as is one that
@@ -1003,8 +1005,10 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 //   f32  1500x3840x1280 137 / 80 (256x96), 1500x5120x1280 165 / 95 (256x128),
 //        1500x1280x5120 162 / 115 and 1500x1280x1280 51 / 33 (128x64x64),
 //        512x4096x1024 40.0 / 29.5, 1024x3072x768 47.1 / 35.3 (64x64),
-//        2048x768x3072 83 / 69; where it loses and stays unpicked: 512x1024x1024
-//        13.7 / 21, 512x384x384 5.1 / 10.5, 256x3072x1024 18.5 / 21 (few tiles);
+//        2048x768x3072 83 / 62; where it loses and stays unpicked: 512x1024x1024
+//        13.4 / 21, 512x1536x384 9.5 / 11.0, 512x384x384 5.1 / 10.5, 256x3072x1024
+//        18.5 / 21 (few tiles); unpicked though level by now: 1500x1536x384 20.4 - 21.2 /
+//        19.7 (64x64);
 //   F16  1500x3840x1280 140 / 69, 1500x1280x5120 169 / 105, 512x4096x1024 40.1 /
 //        27.1, 1500x1536x384 19.7 / 17.8, 391x1536x384 11.2 / 9.8;
 //   Q8_K 1500x3840x1280 159 / 82, 1500x1280x5120 185 / 127, 512x4096x1024 44.7 /
@@ -1012,8 +1016,7 @@ bool gemm_sbf_supported(const MatmulArgs &m) {
 // 2-norm error against 64 bits, the same shapes: 3.7e-7 - 9.9e-7 / 0.9e-7 - 4.5e-7.
 // int8 / int4 (other_us: the plan of gemm_qbf.hip), us: Q8_0 1500x3840x1280 54-58 /
 // 45.3 (256x96), 1500x5120x1280 57-60 / 50.3, 1500x1280x5120 69-73 / 59.6 (256x128, K
-// split 4); back to back in one encoder layer 42.5 / 38.8, 49.2 / 49.0 and 61.5 /
-// 58.1; where it stays unpicked: 1024x4096x1024 28.0 / 32.7, 1500x1280x1280 25.1 / 38.
+// split 4); back to back 42.5 / 39.5, 49.2 / 45.4 and 61.5 / 52.0; where it stays unpicked: 1024x4096x1024 28.0 / 32.7, 1500x1280x1280 25.1 / 38.
 //
 // Layouts no other kernel has wide loads for (K % 4 != 0, odd N, A on a 4-byte
 // boundary) always come here: the register-staged kernel reads them element by
