@@ -137,7 +137,9 @@ int tml_hip_sgemm_q8(int64_t M, int64_t N, int64_t K, const float *A, const int8
  * (M > 8) with an exact three-term split, or, where K % 4 == 0, N % 8 == 0 and the
  * product is small, as everywhere else, on fp32 multiply-adds.  All agree with
  * the reference's dequantize-then-fp32-accumulate result to ~1e-5 relative;
- * infinities and NaNs in A give what the reference gives.  Limit: the
+ * infinities and NaNs in A give what the reference gives (recomputed as described
+ * below at the largest sizes and outside those layouts: up to eight times the time
+ * of a call with none where every output is).  Limit: the
  * per-tensor scale multiplies the finished sum (the reference multiplies
  * each element, a * (q * s)), so finite activations large enough that
  * x * q overflows fp32 (|x| > FLT_MAX / 127 for int8, / 8 for int4) give
@@ -153,8 +155,9 @@ int tml_hip_sgemm_q8(int64_t M, int64_t N, int64_t K, const float *A, const int8
  * bits 1e-7 to 1e-6).  Outputs that the terms cannot carry -- infinities, NaNs,
  * operands past the largest bf16, sums (zero included) that an operand below 2^-102
  * or a product below 2^-80 may have put off by 2^-24 of themselves -- are
- * recomputed from the operands on the fp32 matrix cores, at most five times the time of
- * a call with none. */
+ * recomputed from the operands on the fp32 matrix cores.  A call then takes longer:
+ * about twice its time with one row of NaNs in A, five times where every output is
+ * recomputed. */
 
 /* C = A . dequant(Q8_K B).  Replaces zblas.sgemmQ8K(m, n, k, a, b.data,
  * b.scales, b.block_size, c) at src/core/quantization.zig:555

@@ -199,6 +199,7 @@ __device__ __forceinline__ void sbf_recompute(const SbfArgs &a, float *v, int ro
                         __builtin_amdgcn_raw_buffer_load_b32(rss, k * ((unsigned)a.N / 8u) + col / 32u * 4u, 0, 0));
             }
         }
+        __builtin_amdgcn_sched_barrier(0);  // (all U steps' loads first: the scheduler would spread them, a wait each)
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
