@@ -241,9 +241,9 @@ struct SbfRange {
 // Puts right the outputs in ct, the tile's sums over k in [kbase, kend), that the split
 // does not carry (top of the file).  Small ones are first weighed by what their own
 // row of A and column of B hold: a sum of zeros, or of values that cancel, is as good as
-// any, and rows of zeros are told apart before any column is read.  512x4096x1024 f32 with
-// one column of zeros: 50 us, 29 without (cold instructions, then the loads' latency).  top: the
-// largest magnitude this lane has split.  ex: LDS, sbf_repair_floats floats.
+// any, and rows of zeros are told apart before any column is read.  512x4096x1024 f32
+// with one column of zeros: 50 us, 29 without (cold instructions, then the loads'
+// latency).  top: the largest magnitude this lane has split.  ex: LDS, kSbfRepairFloats.
 template <int BM, int BN, int NW>
 constexpr int kSbfRepairFloats = 2 * (BM + 64 * NW);
 template <int FMT, int BM, int BN, int NW>
@@ -326,7 +326,8 @@ __device__ __forceinline__ void sbf_repair(const SbfArgs &a, float *ct, float *e
                 if (r >= rows || c >= cols || !(fabsf(*v) < doubt)) continue;
                 const SbfRange x = rrow[r], y = rcol[c];
                 if (x.lo == ~0u || y.lo == ~0u) continue;  // a sum of zeros
-                float off = x.least() * y.least() < 0x1p-80f ? kk * 0x1p-98f : 0.0f;  // (2^-23 twice down to the last bits' product)
+                // (the last bits' product is 2^-46 of the values')
+                float off = x.least() * y.least() < 0x1p-80f ? kk * 0x1p-98f : 0.0f;
                 if (x.least() < 0x1p-102f) off += kk * 0x1p-100f * y.most();
                 if (y.least() < 0x1p-102f) off += kk * 0x1p-100f * x.most();
                 if (fabsf(*v) < off) *v = __builtin_nanf("");
